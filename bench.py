@@ -233,8 +233,7 @@ def tuner_record(L, plan, chosen):
     return {"timed": timed, "chosen": pick, "chosen_ms_one_group": tuned, "default": [0, 32, 1],
             "default_ms": default,
             "speedup_vs_default": round(default / tuned, 3) if default and tuned else None,
-            "note": "entries [strip_rows, coh_rows, groups, stage, ms]; stages 1 and 2 eager "
-                    "runs, stage 3 (burst groups) replayed graphs"}
+            "note": "entries [strip_rows, coh_rows, groups, stage, ms]; all stages eager runs"}
 
 
 def issue_fields(roof, kernel, workload, launch_s, samples_per_launch):

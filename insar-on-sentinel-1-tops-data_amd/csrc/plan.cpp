@@ -599,9 +599,14 @@ const char* tops_plan_kernel_name(const tops_plan* p, int kind)
 //      band (3 az x 10 rg window);
 //   2. for a batched schedule with the band form of the coherence, its rows
 //      per block;
-//   3. for a batched schedule, the number of burst groups whose coherence
-//      runs on the second stream beside the next group's resampling (one
-//      group included), timed as replayed graphs.
+//   3. for a batched schedule on the null stream, the number of burst groups
+//      whose coherence runs on the second stream beside the next group's
+//      resampling (one group included).  On a stream of the caller's one group
+//      is kept: there the plan is replayed as a graph, in which groups gain
+//      nothing (27 bursts of 21000 to 25000 columns: 10.70 ms, 10.81 to 10.97
+//      with 2 to 6), and processes that made, launched and at once destroyed the
+//      forked graphs needed to time them have ended with a host segmentation
+//      fault whose cause is not known.  tops_plan_set_groups sets them.
 // It keeps the fastest of each stage and records every candidate timed
 // (tops_plan_tune_entry).  With TOPS_TUNE_CACHE set, the choice is read from
 // / appended to that text file ("<key> <strip_rows> <coh_rows> <groups>"
@@ -628,35 +633,6 @@ int time_runs(tops_plan* p, hipStream_t s, hipEvent_t e0, hipEvent_t e1, float* 
     }
     *out = tot / 3.f;
     return TOPS_OK;
-}
-
-// mean ms per replay of a graph of the plan's current schedule, captured on
-// s (not the null stream), over 3 replays after a warm-up
-int time_graph(tops_plan* p, hipStream_t s, hipEvent_t e0, hipEvent_t e1, float* out)
-{
-    hipGraph_t g = nullptr;
-    hipGraphExec_t x = nullptr;
-    TOPS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue(p, s);
-    hipError_t e = hipStreamEndCapture(s, &g);
-    if (!rc && e != hipSuccess) rc = hip_fail(e, "tops_plan_tune capture", __FILE__, __LINE__);
-    if (!rc && (e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0)) != hipSuccess)
-        rc = hip_fail(e, "tops_plan_tune instantiate", __FILE__, __LINE__);
-    float tot = 0.f;
-    for (int k = -1; k < 3 && !rc; k++) {   // k = -1: warm-up
-        e = hipEventRecord(e0, s);
-        if (e == hipSuccess) e = hipGraphLaunch(x, s);
-        if (e == hipSuccess) e = hipEventRecord(e1, s);
-        if (e == hipSuccess) e = hipEventSynchronize(e1);
-        float ms = 0.f;
-        if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-        if (e != hipSuccess) rc = hip_fail(e, "tops_plan_tune graph timing", __FILE__, __LINE__);
-        if (k >= 0) tot += ms;
-    }
-    if (x) (void)hipGraphExecDestroy(x);
-    if (g) (void)hipGraphDestroy(g);
-    if (!rc) *out = tot / 3.f;
-    return rc;
 }
 
 }  // namespace
@@ -764,25 +740,19 @@ int tops_plan_tune(tops_plan* p, void* stream, int* best_rows)
         p->coh_rows = best_c;
         if (!rc) rc = fill_coh_work(p);
     }
-    // stage 3: burst groups pipelined over two streams (batched schedule),
-    // one group included, timed as replayed graphs when the caller's stream
-    // can capture one (the overlap of the two streams is not the same in a
-    // graph as in eager launches: 9 groups of the IW pair measured 11.7 ms
-    // eager and 12.5 ms replayed, so graphs decide, and the search stops at
-    // 6 groups)
+    // stage 3: burst groups pipelined over two streams (batched schedule)
     if (!rc && best_r > 0 && p->coh_batched && p->items.size() > 1) {
         int best_g = 1;
         float best3 = 1e30f;
-        std::vector<int> gs;
-        for (int g : {1, 2, 3, 4, 6})
-            if (g <= (int)p->items.size() && std::find(gs.begin(), gs.end(), g) == gs.end())
-                gs.push_back(g);
+        std::vector<int> gs = {1};
+        for (int g : {2, 3, 4, 6})
+            if (!s && g <= (int)p->items.size()) gs.push_back(g);
         for (int g : gs) {
             p->groups = g;
             partition(p);
             float ms = 0.f;
             if ((rc = ensure_pipe(p)) || (rc = fill_work(p)) || (rc = fill_coh_work(p)) ||
-                (rc = s ? time_graph(p, s, e0, e1, &ms) : time_runs(p, s, e0, e1, &ms)))
+                (rc = time_runs(p, s, e0, e1, &ms)))
                 break;
             p->tune_log.push_back({best_r, p->coh_rows, g, 3, ms});
             if (ms < best3) {

@@ -1,0 +1,80 @@
+"""Host side of the library on a stand-in HIP runtime (hip_stub.cpp): which
+calls it makes, with which tables, and what it does when one fails.  Each test
+runs a short program of its own in a process that preloads the stand-in, so
+nothing here needs a GPU."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import PKG_DIR
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes as C, numpy as np, sys
+sys.modules["torch"] = None          # the bindings then load without it
+import importlib.util
+spec = importlib.util.spec_from_file_location("native", {native!r})
+N = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(N)
+L = N.load()
+S = C.CDLL({stub!r})
+S.stub_count.restype = S.stub_bad.restype = S.stub_host_blocks.restype = C.c_long
+S.stub_fail.argtypes = [C.c_char_p, C.c_long]
+S.stub_device_bytes.restype = C.c_size_t
+count = lambda what: S.stub_count(what.encode())
+lut = np.full(2048 * 12, 1 / 12, np.float32)
+ctx = L.tops_ctx_create(N.ptr(lut, C.c_float), N.ptr(lut, C.c_float), 12)
+FAKE = 0x10000000                    # a device address: no kernel runs
+
+def geom(lines, pixels):
+    g = N.BurstGeom()
+    g.master_box[:] = g.slave_box[:] = [0, pixels - 1, 0, lines - 1]
+    g.samples_per_burst, g.az_time_interval = pixels, 2e-3
+    g.cpm_az[:] = [lines / 2, lines / 4, 0, 0, 0, 0]
+    g.cpm_rg[:] = [pixels / 2, 0, pixels / 4, 0, 0, 0]
+    return g
+
+def plan(shapes, win=(3, 10), strip_rows=0):
+    items = (N.BurstItem * len(shapes))(*[N.BurstItem(geom(h, w), *[FAKE] * 7) for h, w in shapes])
+    p = L.tops_plan_create(ctx, items, len(shapes), win[0], win[1], strip_rows)
+    assert p, N.last_error()
+    return p
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    stub = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-w", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_stub.cpp"), "-o", stub], check=True)
+    prelude = PRELUDE.format(native=os.path.join(PKG_DIR, "native.py"), stub=stub)
+
+    def program(text):
+        r = subprocess.run([sys.executable, "-c", prelude + text], capture_output=True, text=True,
+                           timeout=300, env=dict(os.environ, LD_PRELOAD=stub))
+        assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
+        return r.stdout
+
+    return program
+
+
+TUNE = """
+p = plan([(300 + 40 * i, 2500 + 300 * i) for i in range(7)])
+stream = C.c_void_p()
+S.hipStreamCreate(C.byref(stream))
+best = C.c_int()
+N.check(L.tops_plan_tune(p, stream, C.byref(best)))
+"""
+
+
+def test_tune_makes_no_graph(run):
+    """Tuning times eager launches: no graph is made, launched and destroyed
+    while the plan is being formed."""
+    run(TUNE + """
+assert L.tops_plan_tune_count(p) > 10 and count("hipGraphInstantiate") == 0
+N.check(L.tops_plan_capture_graph(p, stream))
+assert count("hipGraphInstantiate") == 1 and S.stub_bad() == 0
+""")
