@@ -246,7 +246,7 @@ int tops_plan_capture_graph(tops_plan* plan, void* stream);
  * named by TOPS_TUNE_CACHE when set. */
 int tops_plan_tune(tops_plan* plan, void* stream, int* best_strip_rows);
 int tops_plan_strip_rows(const tops_plan* plan);
-/* Rows per block of the plan's batched coherence walk (default 32). */
+/* Rows per block of the plan's batched coherence launch (default 32). */
 int tops_plan_coh_rows(const tops_plan* plan);
 /* Burst groups of the batched schedule (default 1): the bursts split into
  * that many runs of consecutive bursts with about equal sample counts; each

@@ -19,7 +19,7 @@
 
 using namespace tops;
 
-constexpr int kDefaultCohRows = 32;   // coh_rows before tuning: the band rows by rule
+constexpr int kDefaultCohRows = 32;   // coh_rows before tuning
 
 struct tops_plan {
     tops_ctx* ctx = nullptr;
@@ -44,11 +44,7 @@ struct tops_plan {
     // schedule forms coherence with one launch per burst
     bool coh_batched = true;
     CohForm coh_form = CohForm::kDirect;   // of the batched launch
-    // output rows per block of the batched band launch; kDefaultCohRows stands
-    // for the height coherence_band_rows gives the batch (band_rows0)
-    int coh_rows = kDefaultCohRows;
-    int band_rows0 = kDefaultCohRows;
-    int band_rows() const { return coh_rows == kDefaultCohRows ? band_rows0 : coh_rows; }
+    int coh_rows = kDefaultCohRows;   // output rows per block of the batched band launch
     // batched schedule in burst groups: group g (items grp_first[g] ..
     // grp_first[g+1]-1) is resampled by one launch on the caller's stream,
     // and its coherence launch on a second stream waits for that launch
@@ -180,9 +176,6 @@ int fill_params(tops_plan* p)
     p->coh_form = coherence_form(cw.data(), ch.data(), nc, (p->coh_win_rg - 1) / 2,
                                  (p->coh_win_az - 1) / 2, p->coh_win_rg, p->coh_win_az);
     p->coh_batched = p->coh_form != CohForm::kDirect;
-    if (p->coh_form == CohForm::kBand && nc)
-        p->band_rows0 =
-            coherence_band_rows(cw.data(), ch.data(), nc, p->coh_win_rg, p->coh_win_az);
     p->coh_item.assign(ci.size(), 0);
     for (size_t i = 0; i < p->items.size(); i++)
         if (p->coh_of[i] >= 0) p->coh_item[p->coh_of[i]] = (int)i;
@@ -214,7 +207,7 @@ int fill_params(tops_plan* p)
 }
 
 // work table of the batched coherence launch: {coherence item, column band,
-// row block, 0}, blocks of band_rows() rows for the band form, 16 x 64 tiles
+// row block, 0}, blocks of coh_rows rows for the band form, 16 x 64 tiles
 // otherwise
 int fill_coh_work(tops_plan* p)
 {
@@ -231,7 +224,7 @@ int fill_coh_work(tops_plan* p)
             const CohItem& c = p->h_coh[k];
             int nx, ny;
             if (p->coh_form == CohForm::kBand)
-                coherence_band_count(c.w, c.h, p->coh_win_rg, p->band_rows(), &nx, &ny);
+                coherence_band_count(c.w, c.h, p->coh_win_rg, p->coh_rows, &nx, &ny);
             else
                 coherence_tile_count(c.w, c.h, &nx, &ny);
             for (int y = 0; y < ny; y++)
@@ -399,7 +392,7 @@ int enqueue(tops_plan* p, hipStream_t s, Marks* mk = nullptr)
             TOPS_HIP(hipStreamWaitEvent(p->s2, p->ev_grp[g], 0));
             rc = marked(mk, p->s2, kKindCoherence, [&] {
                 return launch_coherence_batch(p->d_coh, p->d_work_coh + c0, nc, p->coh_form, dx,
-                                              dy, p->coh_win_rg, p->coh_win_az, p->band_rows(), p->s2);
+                                              dy, p->coh_win_rg, p->coh_win_az, p->coh_rows, p->s2);
             });
         }
         // the caller's stream waits for the coherence stream (also when a
@@ -417,7 +410,7 @@ int enqueue(tops_plan* p, hipStream_t s, Marks* mk = nullptr)
     if (p->coh_batched)
         return marked(mk, s, kKindCoherence, [&] {
             return launch_coherence_batch(p->d_coh, p->d_work_coh, p->n_work_coh, p->coh_form,
-                                          dx, dy, p->coh_win_rg, p->coh_win_az, p->band_rows(), s);
+                                          dx, dy, p->coh_win_rg, p->coh_win_az, p->coh_rows, s);
         });
     for (const CohItem& c : p->h_coh)
         if ((rc = coh_one(c))) return rc;
@@ -711,8 +704,9 @@ int tops_plan_tune(tops_plan* p, void* stream, int* best_rows)
     TOPS_HIP(hipEventCreate(&e0));
     TOPS_HIP(hipEventCreate(&e1));
     drop_graph(p);
-    int rc = TOPS_OK;
+    int rc = fill_coh_work(p);   // (an earlier tuning's table is of its own height)
     for (int c : cand) {
+        if (rc) break;
         p->strip_rows = c;
         float ms = 0.f;
         if ((rc = fill_work(p)) || (rc = time_runs(p, s, e0, e1, &ms))) break;

@@ -78,3 +78,30 @@ assert L.tops_plan_tune_count(p) > 10 and count("hipGraphInstantiate") == 0
 N.check(L.tops_plan_capture_graph(p, stream))
 assert count("hipGraphInstantiate") == 1 and S.stub_bad() == 0
 """)
+
+
+def test_coherence_rows_are_the_launched_ones(run):
+    """tops_plan_coh_rows and the tuner's entries give the height the batched
+    coherence was launched with, 32 included, also in a second tuning."""
+    run("""
+p = plan([(300 + 40 * i, 2500 + 300 * i) for i in range(7)], strip_rows=64)
+N.check(L.tops_plan_run(p, None))
+assert S.stub_band_rows() == L.tops_plan_coh_rows(p) == 32 and S.stub_bad() == 0
+best = C.c_int()
+for _ in range(2):
+    N.check(L.tops_plan_tune(p, None, C.byref(best)))
+    assert S.stub_bad() == 0
+    N.check(L.tops_plan_run(p, None))
+    if best.value > 0:
+        assert S.stub_band_rows() == L.tops_plan_coh_rows(p)
+    # the next tuning starts from a table of another height
+    N.check(L.tops_plan_set_groups(p, 1))
+""" + """
+timed = []
+for i in range(L.tops_plan_tune_count(p)):
+    v = [C.c_int() for _ in range(4)]
+    ms = C.c_float()
+    N.check(L.tops_plan_tune_entry(p, i, *[C.byref(x) for x in v], C.byref(ms)))
+    timed.append([x.value for x in v])
+assert {e[1] for e in timed if e[3] == 2} <= {16, 64, 128, 256} and 32 in {e[1] for e in timed}
+""")
