@@ -19,12 +19,12 @@
 // magnitudes, and the same for every split into bands and row blocks (bands
 // start at multiples of 4 columns).
 // What bounds it: memory for windows of up to 7 lines (1500 x 21000, 0.5 GB:
-// 98-110 us, 5.1 TB/s at 3 lines), waves in flight above (8 lines, 205 VGPRs: 2
+// 97-105 us, 5.1 TB/s at 3 lines), waves in flight above (8 lines, 205 VGPRs: 2
 // waves per SIMD).  Against the tiles, whose LDS traffic and halo bound them, on 1500 x
-// 21000 / 1487 x 24491, us: 5 x 20 183 / 214 -> 101 / 116, 6 x 24 153 / 174 ->
-// 104 / 117, 8 x 32 286 / 334 -> 122 / 135, 4 x 9 161 / 188 -> 99 / 114, 2 x 8
-// 223 / 262 -> 98 / 124.  Against one row of products at a time in LDS for a
-// fixed 3 x 10 window, 2 columns per thread: 95 / 130 -> 99 / 113, 42 -> 34 on
+// 21000 / 1487 x 24491, us: 5 x 20 183 / 214 -> 100 / 116, 6 x 24 153 / 174 ->
+// 105 / 117, 8 x 32 286 / 334 -> 131 / 144, 4 x 9 161 / 188 -> 96 / 114, 2 x 8
+// 223 / 262 -> 96 / 123.  Against one row of products at a time in LDS for a
+// fixed 3 x 10 window, 2 columns per thread: 95 / 130 -> 97 / 113, 42 -> 35 on
 // 1400 x 9000.
 #pragma once
 
@@ -59,24 +59,29 @@ struct BandSum {
 };
 
 // Azimuth sums over the WA latest rows.  push(p, q) takes row number q (mod
-// kPeriod, a compile-time constant after unrolling) and returns the sum.  The
-// terms are added in an order that depends neither on q nor on which end of
-// the window came first, so a walk up and a walk down give the same bits.
+// kPeriod, a compile-time constant after unrolling) and returns the sum: rows
+// a steps from the two ends in pairs, pairs in two halves.  The order depends
+// neither on q nor on which end of the window came first, so a walk up and a
+// walk down give the same bits.
 template <int WA>
 struct BandColumns {
     static constexpr int kPeriod = WA - 1;   // direct: the WA - 1 rows before this one
+    static_assert(WA <= CB_MAX_AZ, "up to four terms");
     BandSum ring[WA - 1];
     __device__ __forceinline__ BandSum push(const BandSum& p, int q)
     {
         constexpr int D = WA - 1;
-        BandSum s = p + ring[q % D];   // the oldest
+        constexpr int N = (WA + 1) / 2;   // terms: pairs, and the middle row of an odd WA
+        const BandSum ends = p + ring[q % D];   // with the oldest
         ring[q % D] = p;
-#pragma unroll
-        for (int a = 1; a < (WA + 1) / 2; a++) {
+        auto term = [&](int a) {
             const BandSum& y = ring[(q + D - a) % D];
-            s = 2 * a == D ? s + y : s + (y + ring[(q + a) % D]);
-        }
-        return s;
+            return 2 * a == D ? y : y + ring[(q + a) % D];
+        };
+        if constexpr (N == 1) return ends;
+        else if constexpr (N == 2) return ends + term(1);
+        else if constexpr (N == 3) return ends + (term(1) + term(2));
+        else return (ends + term(1)) + (term(2) + term(3));
     }
 };
 // pairs S2(r) = P(r) + P(r - 1): 4 lines are S2(r) + S2(r - 2)
@@ -230,14 +235,24 @@ struct BandRange {
         }
     }
     // f(j, sums of the window at column j), j = 3 .. 0: one window at a time,
-    // so that few sums are held at once
+    // so that few sums are held at once.  The window's ends are added to each
+    // other and only then to its middle, which is two chains: few of the sums
+    // are rounded at the size of the whole.  (RMS error of the coherence against
+    // 64 bits, 6 x 24 / 8 x 32 windows: 5.4e-8 / 5.5e-8; 5.9e-8 / 6.2e-8 with
+    // one chain from left to right, 5.5e-8 / 5.7e-8 in the tiles.)
     template <class F>
     __device__ __forceinline__ void sums(const BandSum& V, const float4* E, int t, F&& f) const
     {
         const float4* T = E + 3 * NT + t;
-        float4 mid = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 4
-        for (int k = 1; k < kmin; k++) mid = add4(mid, T[k]);
+        float4 mid = make_float4(0.f, 0.f, 0.f, 0.f), odd = mid;
+        int k = 1;
+#pragma unroll 2
+        for (; k + 1 < kmin; k += 2) {
+            mid = add4(mid, T[k]);
+            odd = add4(odd, T[k + 1]);
+        }
+        if (k < kmin) mid = add4(mid, T[k]);   // (uniform)
+        mid = add4(mid, odd);
         __builtin_amdgcn_sched_barrier(0);
         float4 tail[CB_PER_THREAD], x = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
@@ -247,12 +262,12 @@ struct BandRange {
 #pragma unroll
         for (int j = CB_PER_THREAD - 1; j >= 0; j--) {
             if (j < CB_PER_THREAD - 1) s = add4(band_col(V, j), s);
-            float4 o = add4(s, mid);
+            float4 o = s;
             // (uniform branches)
+            if (j > 0 || a) o = add4(o, tail[j]);
             if (j == 3 && a >= 2) o = add4(o, x);
             if (j == 2 && a == 3) o = add4(o, x);
-            if (j > 0 || a) o = add4(o, tail[j]);
-            f(j, o);
+            f(j, add4(o, mid));
             __builtin_amdgcn_sched_barrier(0);
         }
     }
