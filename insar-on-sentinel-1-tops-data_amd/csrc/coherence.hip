@@ -20,7 +20,6 @@
 
 #include <algorithm>
 #include <type_traits>
-#include <vector>
 
 namespace tops {
 
@@ -159,13 +158,15 @@ coherence_band_batch_kernel(const CohItem* items, const int4* work, int dx, int 
                        by & 1, smem);
 }
 
-// The form of a launch over n rasters of one window.  A band's workgroup is a
+// The form of a launch over n rasters of one window (sizes w[i * step], h[i *
+// step]; step 0: all of one size).  A band's workgroup is a
 // chain of its rows and the window's, so rasters whose tiles all run at once
 // stay with them: up to 4 tiles per CU for windows of up to 5 lines, 8 above
 // (us, tiles against bands, 256 CUs: 3 x 10 window 6.6 / 7.3 on 512 x 2048,
 // 8.2 / 7.7 on 600 x 2000, 13.5 / 9.1 on 700 x 3000; 6 x 24 window 11.9 / 14.5
 // on 1500 x 1100, 14.6 / 13.5 on 700 x 3000, 153 / 102 on 1500 x 21000).
-CohForm coherence_form(const int* w, const int* h, int n, int dx, int dy, int win_rg, int win_az)
+CohForm coherence_form(const int* w, const int* h, int n, int step, int dx, int dy, int win_rg,
+                       int win_az)
 {
     const bool tile_ok = tile_window_launch_lds(win_rg, win_az) != 0;
     bool band_ok = win_az >= 2 && win_az <= CB_MAX_AZ && win_rg >= CB_PER_THREAD &&
@@ -173,8 +174,8 @@ CohForm coherence_form(const int* w, const int* h, int n, int dx, int dy, int wi
     long tiles = 0;
     for (int i = 0; i < n; i++) {
         int nx, ny;
-        tiles += coherence_tile_count(w[i], h[i], &nx, &ny);
-        band_ok = band_ok && w[i] <= CB_MAX_WIDTH;
+        tiles += coherence_tile_count(w[i * step], h[i * step], &nx, &ny);
+        band_ok = band_ok && w[i * step] <= CB_MAX_WIDTH;
     }
     if (band_ok && (!tile_ok || tiles > (long)device_cus() * (win_az <= 5 ? 4 : 8)))
         return CohForm::kBand;
@@ -193,28 +194,23 @@ int coherence_band_count(int w, int h, int win_rg, int rows, int* nx, int* ny)
 // CU for 3 to 7 lines (a fourth fits beside 3 lines but reads more halo rows:
 // 101 us instead of 99 on 1500 x 21000), else as many as fit (2 lines: 103 us
 // with 4, 114 with 3).  Launches of many rasters take further rounds rather
-// than more than 96 rows.
-int coherence_band_rows(const int* w, const int* h, int n, int win_rg, int win_az)
+// than more than 96 rows, up to the 65535 row blocks a grid has.
+static int coherence_band_rows(int w, int h, int n, int win_rg, int win_az)
 {
     const long slots = (long)device_cus() * (win_az == 3 ? 3 : band_waves(win_az));
-    int hmax = 1;
-    for (int i = 0; i < n; i++) hmax = std::max(hmax, h[i]);
+    const int least = (int)((h + 65534l) / 65535);
     for (long round = 1;; round++) {
-        int lo = 1, hi = hmax;   // the smallest height within `round` rounds
+        int lo = 1, hi = h;   // the smallest height within `round` rounds
         auto blocks = [&](int rows) {
-            long t = 0;
-            for (int i = 0; i < n; i++) {
-                int nx, ny;
-                t += coherence_band_count(w[i], h[i], win_rg, rows, &nx, &ny);
-            }
-            return t;
+            int nx, ny;
+            return (long)n * coherence_band_count(w, h, win_rg, rows, &nx, &ny);
         };
         while (lo < hi) {
             const int mid = (lo + hi) / 2;
             if (blocks(mid) <= round * slots) hi = mid;
             else lo = mid + 1;
         }
-        if (lo <= 96 && blocks(lo) <= round * slots) return lo;
+        if (lo <= 96 && blocks(lo) <= round * slots) return std::max(lo, least);
     }
 }
 
@@ -257,8 +253,7 @@ int launch_coherence_batch(const CohItem* d_items, const int4* d_work, int n_wor
 static int launch_band(const tops_ci16* m, const tops_cf32* s, int w, int h, int n, size_t stride,
                        int dx, int dy, int win_rg, int win_az, float* coh, hipStream_t st)
 {
-    const std::vector<int> ws(n, w), hs(n, h);
-    const int rows = coherence_band_rows(ws.data(), hs.data(), n, win_rg, win_az);
+    const int rows = coherence_band_rows(w, h, n, win_rg, win_az);
     int nx, ny;
     coherence_band_count(w, h, win_rg, rows, &nx, &ny);
     band_dispatch(win_az, [&](auto wa) {
@@ -276,9 +271,7 @@ int launch_coherence_stack(const tops_ci16* m, const tops_cf32* s, int w, int h,
 {
     // bands of all rasters in one launch (9 of 1500 x 23500, 6 x 24: 1.01 ms
     // against 1.08 one by one)
-    const std::vector<int> ws(n, w), hs(n, h);
-    if (coherence_form(ws.data(), hs.data(), n, dx, dy, win_rg, win_az) == CohForm::kBand &&
-        n <= 65535)
+    if (coherence_form(&w, &h, n, 0, dx, dy, win_rg, win_az) == CohForm::kBand && n <= 65535)
         return launch_band(m, s, w, h, n, stride, dx, dy, win_rg, win_az, coh, st);
     int rc = TOPS_OK;
     for (int i = 0; i < n && !rc; i++)
@@ -292,7 +285,7 @@ int launch_coherence(const tops_ci16* m, const tops_cf32* s, int w, int h, int d
 {
     const CohForm form = mode == TOPS_MODE_FP64
                              ? CohForm::kDirect
-                             : coherence_form(&w, &h, 1, dx, dy, win_rg, win_az);
+                             : coherence_form(&w, &h, 1, 0, dx, dy, win_rg, win_az);
     if (form == CohForm::kBand)
         return launch_band(m, s, w, h, 1, 0, dx, dy, win_rg, win_az, coh, st);
     if (form == CohForm::kDirect) {

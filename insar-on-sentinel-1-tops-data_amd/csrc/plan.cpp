@@ -173,7 +173,7 @@ int fill_params(tops_plan* p)
         ch.push_back(c.h);
     }
     const int nc = (int)ci.size();
-    p->coh_form = coherence_form(cw.data(), ch.data(), nc, (p->coh_win_rg - 1) / 2,
+    p->coh_form = coherence_form(cw.data(), ch.data(), nc, 1, (p->coh_win_rg - 1) / 2,
                                  (p->coh_win_az - 1) / 2, p->coh_win_rg, p->coh_win_az);
     p->coh_batched = p->coh_form != CohForm::kDirect;
     p->coh_item.assign(ci.size(), 0);
@@ -572,7 +572,7 @@ const char* tops_plan_kernel_name(const tops_plan* p, int kind)
         // (the first burst's form)
         CohForm f = CohForm::kDirect;
         if (!p->h_coh.empty())
-            f = coherence_form(&p->h_coh[0].w, &p->h_coh[0].h, 1, (p->coh_win_rg - 1) / 2,
+            f = coherence_form(&p->h_coh[0].w, &p->h_coh[0].h, 1, 0, (p->coh_win_rg - 1) / 2,
                                (p->coh_win_az - 1) / 2, p->coh_win_rg, p->coh_win_az);
         return f == CohForm::kDirect ? "coherence_fp64_kernel"
                : f == CohForm::kBand ? "coherence_band_kernel"

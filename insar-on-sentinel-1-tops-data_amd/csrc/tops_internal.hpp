@@ -221,14 +221,14 @@ struct CohItem {
 // how a launch forms its window sums: FP64 per output, 16 x 64 tiles in LDS, or
 // bands of columns walked down (coherence_band.hpp)
 enum class CohForm { kDirect, kTile, kBand };
-CohForm coherence_form(const int* w, const int* h, int n, int dx, int dy, int win_rg, int win_az);
+CohForm coherence_form(const int* w, const int* h, int n, int step, int dx, int dy, int win_rg,
+                       int win_az);
 // batched work items are {item, column band, row block of band_rows output
 // rows, 0} (kBand) or {item, tile x, tile y, 0} (kTile)
 int launch_coherence_batch(const CohItem* d_items, const int4* d_work, int n_work, CohForm form,
                            int dx, int dy, int win_rg, int win_az, int band_rows, hipStream_t st);
 int coherence_tile_count(int w, int h, int* nx, int* ny);
 int coherence_band_count(int w, int h, int win_rg, int rows, int* nx, int* ny);
-int coherence_band_rows(const int* w, const int* h, int n, int win_rg, int win_az);
 
 // launchers (fused.hip): one persistent launch of deramp -> resample ->
 // reramp -> coherence over work items {burst, column strip, first row, rows}

@@ -105,3 +105,13 @@ for i in range(L.tops_plan_tune_count(p)):
     timed.append([x.value for x in v])
 assert {e[1] for e in timed if e[3] == 2} <= {16, 64, 128, 256} and 32 in {e[1] for e in timed}
 """)
+
+
+def test_coherence_of_very_long_narrow_rasters(run):
+    """A raster of more row blocks than a grid has rows is launched with taller
+    blocks (3 x 10 windows, one column band)."""
+    run("""
+for lines in (6_200_000, 6_300_000, 40_000_000):
+    N.check(L.tops_coherence(FAKE, FAKE, 5, lines, 4, 1, 10, 3, FAKE, N.MODE_FAST, None))
+    assert S.stub_bad() == 0, lines
+""")
