@@ -14,7 +14,7 @@
 // Each call is ordered after the work already queued on the null stream (the
 // stage layer's launches) and returns when its copies are complete, so it
 // replaces a synchronous hipMemcpy.  Buffers the runtime knows (pinned,
-// managed) and short ones are left to hipMemcpy, as is everything when the
+// managed) and short ones are left to hipMemcpy, as is everything while the
 // pool cannot be made.  The pool of each device (64 MiB pinned, one stream, two
 // events) is made on first use and kept until the process ends; calls on one
 // device are serialised by its lock.
@@ -37,7 +37,7 @@ constexpr int kThreads = 8;
 
 struct Pool {
     std::mutex mu;
-    bool ready = false, failed = false;
+    bool ready = false;
     char* buf[2] = {nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipStream_t s = nullptr;
@@ -45,17 +45,35 @@ struct Pool {
 
 Pool g_pools[kMaxDevices];
 
+// whether the runtime knows the memory: pinned, managed or device memory, not
+// malloc'd, stack or mapped files
+bool known(const void* h)
+{
+    hipPointerAttribute_t a;
+    memset(&a, 0, sizeof(a));
+    if (hipPointerGetAttributes(&a, h) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
+// The pool's buffers, made on first use.  A pool that cannot be made is tried again by the next call.
 bool pool_init(Pool& p)
 {
-    if (p.ready || p.failed) return p.ready;
+    if (p.ready) return true;
+    p.s = nullptr;
+    for (int k = 0; k < 2; k++) {
+        p.buf[k] = nullptr;
+        p.ev[k] = nullptr;
+    }
     hipError_t e = hipStreamCreateWithFlags(&p.s, hipStreamNonBlocking);
     for (int k = 0; k < 2; k++) {
         if (e == hipSuccess) e = hipHostMalloc((void**)&p.buf[k], kMaxChunk, hipHostMallocDefault);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&p.ev[k], hipEventDisableTiming);
     }
     p.ready = e == hipSuccess;
-    p.failed = !p.ready;
-    if (p.failed) {   // give back what was made, and forget the error
+    if (!p.ready) {   // give back what was made, and forget the error
         for (int k = 0; k < 2; k++) {
             if (p.ev[k]) (void)hipEventDestroy(p.ev[k]);
             if (p.buf[k]) (void)hipHostFree(p.buf[k]);
@@ -64,18 +82,6 @@ bool pool_init(Pool& p)
         (void)hipGetLastError();
     }
     return p.ready;
-}
-
-// memory the runtime does not know: malloc'd, stack, mapped files
-bool pageable(const void* h)
-{
-    hipPointerAttribute_t a;
-    memset(&a, 0, sizeof(a));
-    if (hipPointerGetAttributes(&a, h) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return a.type == hipMemoryTypeUnregistered;
 }
 
 // f(0) .. f(n - 1) on threads of their own, the first and those that no thread
@@ -218,7 +224,7 @@ int staged_upload(void* d_dst, const void* h_src, size_t bytes)
 {
     if (bytes == 0) return TOPS_OK;
     int rc = TOPS_OK;
-    if (bytes > kMinChunk && pageable(h_src) &&
+    if (bytes > kMinChunk && !known(h_src) &&
         staged_copy(true, (char*)d_dst, (char*)const_cast<void*>(h_src), bytes, &rc))
         return rc;
     TOPS_HIP(hipMemcpy(d_dst, h_src, bytes, hipMemcpyHostToDevice));
@@ -229,7 +235,7 @@ int staged_download(void* h_dst, const void* d_src, size_t bytes)
 {
     if (bytes == 0) return TOPS_OK;
     int rc = TOPS_OK;
-    if (bytes > kMinChunk && pageable(h_dst) &&
+    if (bytes > kMinChunk && !known(h_dst) &&
         staged_copy(false, (char*)const_cast<void*>(d_src), (char*)h_dst, bytes, &rc))
         return rc;
     TOPS_HIP(hipMemcpy(h_dst, d_src, bytes, hipMemcpyDeviceToHost));

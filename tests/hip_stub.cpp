@@ -10,9 +10,11 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <chrono>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 namespace {
@@ -26,6 +28,7 @@ struct State {
     long bad = 0;
     int band_rows = 0;   // of the last batched band coherence
     bool capturing = false;
+    int sync_ms = 0;     // what a stream synchronisation takes
 };
 State& st()
 {
@@ -95,6 +98,15 @@ long stub_count(const char* what) { return st().count[what]; }
 void stub_fail(const char* what, long nth) { st().fail[what] = nth; }
 long stub_bad() { return st().bad; }
 int stub_band_rows() { return st().band_rows; }
+void stub_sync_ms(int ms) { st().sync_ms = ms; }
+// what hipDeviceReset does to the memory of the device
+void stub_reset()
+{
+    std::lock_guard<std::recursive_mutex> l(st().mu);
+    st().dev.clear();
+    st().host.clear();
+    st().dev_bytes = 0;
+}
 size_t stub_device_bytes() { return st().dev_bytes; }
 long stub_host_blocks() { return (long)st().host.size(); }
 
@@ -205,6 +217,9 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k)
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t)
 {
     if (called("hipMemcpyAsync")) return hipErrorUnknown;
+    if (std::lock_guard<std::recursive_mutex> l(st().mu);
+        k == hipMemcpyHostToDevice && !inside(st().host, s, n))
+        bad("asynchronous upload of memory that is not pinned");
     return hipMemcpy(d, s, n, k);
 }
 hipError_t hipMemset(void* d, int v, size_t n)
@@ -232,7 +247,11 @@ hipError_t hipStreamDestroy(hipStream_t s)
     free(s);
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    std::this_thread::sleep_for(std::chrono::milliseconds(st().sync_ms));
+    return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e)
 {
@@ -293,6 +312,10 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, 
     const std::string& name = st().kernel[f];
     if (name.find("coherence_band_batch_kernel") != std::string::npos)
         check_band_batch(args, grid.x);
+    if (name.find("esd_final_kernel") != std::string::npos ||
+        name.find("geocoreg_final_kernel") != std::string::npos)
+        if (void* out = *(void**)args[2]; !inside(st().dev, out, 48) && !inside(st().host, out, 48))
+            bad("sums written to memory that is not there");
     return hipSuccess;
 }
 

@@ -115,3 +115,34 @@ for lines in (6_200_000, 6_300_000, 40_000_000):
     N.check(L.tops_coherence(FAKE, FAKE, 5, lines, 4, 1, 10, 3, FAKE, N.MODE_FAST, None))
     assert S.stub_bad() == 0, lines
 """)
+
+
+CALLS = """
+import threading
+def esd(lines=40, pixels=900):
+    n = np.full(3, lines, np.int32)
+    sh, su = np.zeros(3), np.zeros(6)
+    N.check(L.tops_esd_shifts(*[FAKE] * 4, N.ptr(n, C.c_int), 3, pixels, 6, 24, 0.3, 5e3, 2e-3,
+                              N.ptr(sh), N.ptr(su), None))
+
+co = np.array([7e6, 1.0, 0, 0, 0, 0])
+og = N.OrbitGeom(*[N.ptr(co)] * 3, 6, 0.0, 2e-3, 0.0, 5e-3, 2.3, 0.0, 0)
+def geocoreg(lines, pixels):
+    a, r = np.zeros(6), np.zeros(6)
+    # (no kernel runs: the sums are not positive definite)
+    rc = L.tops_geocoreg(FAKE, lines, pixels, 45.0, 10.0, 3e-4, 3e-4, -32768, C.byref(og),
+                         C.byref(og), 0, 99, 0, 99, N.ptr(a), N.ptr(r), None, None, None)
+    assert rc in (0, N.TOPS_ERR_NOT_PD), rc
+"""
+
+
+def test_staging_pool_is_tried_again(run):
+    """A pool that could not be made leaves a copy to the runtime, once."""
+    run(CALLS + """
+S.stub_fail(b"hipHostMalloc", 1)
+x = np.zeros(2000 * 900, np.complex64)       # 14.4 MB
+L.ResampleFirstBurst(x.ctypes.data, 900, 2000)
+assert L.tops_last_error() == 0 and count("hipMemcpyAsync") == 0 and S.stub_host_blocks() == 0
+L.ResampleFirstBurst(x.ctypes.data, 900, 2000)
+assert L.tops_last_error() == 0 and count("hipMemcpyAsync") > 0 and S.stub_host_blocks() == 2
+""")
