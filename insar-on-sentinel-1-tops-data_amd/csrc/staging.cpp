@@ -25,7 +25,6 @@
 #include <algorithm>
 #include <mutex>
 #include <thread>
-#include <vector>
 
 namespace tops {
 namespace {
@@ -165,10 +164,42 @@ constexpr size_t kPinnedBytes = 4096;
 
 struct ScratchPool {
     std::mutex mu;
-    std::vector<CallScratch::Block> idle;
+    CallScratch::Block idle[kKeepBlocks];
+    int n = 0;
+
+    CallScratch::Block remove(int i)
+    {
+        const CallScratch::Block b = idle[i];
+        idle[i] = idle[--n];
+        return b;
+    }
+    // the smallest idle block of at least that many bytes, or none
+    CallScratch::Block best(size_t bytes)
+    {
+        int at = -1;
+        for (int i = 0; i < n; i++)
+            if (idle[i].bytes >= bytes && (at < 0 || idle[i].bytes < idle[at].bytes)) at = i;
+        return at < 0 ? CallScratch::Block() : remove(at);
+    }
+    // keeps b, in the place of the smallest block when there is none free; the
+    // block that is not kept (none: nothing)
+    CallScratch::Block keep(const CallScratch::Block& b)
+    {
+        CallScratch::Block out;
+        if (n == kKeepBlocks) {
+            int at = 0;
+            for (int i = 1; i < n; i++)
+                if (idle[i].bytes < idle[at].bytes) at = i;
+            if (idle[at].bytes >= b.bytes) return b;
+            out = remove(at);
+        }
+        idle[n++] = b;
+        return out;
+    }
 };
 ScratchPool g_scratch[kMaxDevices];
 
+// (waits for the device)
 void free_block(const CallScratch::Block& b)
 {
     if (b.dev) (void)hipFree(b.dev);
@@ -179,24 +210,20 @@ void free_block(const CallScratch::Block& b)
 
 int CallScratch::take(size_t dev_bytes, size_t host_bytes)
 {
-    if (hipGetDevice(&device_) != hipSuccess) device_ = -1;
-    if (device_ >= 0 && device_ < kMaxDevices && host_bytes <= kPinnedBytes) {
+    if (hipGetDevice(&device_) != hipSuccess || device_ >= kMaxDevices) device_ = -1;
+    if (device_ >= 0 && dev_bytes <= kKeepBytes && host_bytes <= kPinnedBytes) {
         ScratchPool& p = g_scratch[device_];
         std::lock_guard<std::mutex> lock(p.mu);
-        for (size_t i = 0; i < p.idle.size(); i++)
-            if (p.idle[i].bytes >= dev_bytes) {
-                b_ = p.idle[i];
-                p.idle[i] = p.idle.back();
-                p.idle.pop_back();
-                return TOPS_OK;
-            }
+        if ((b_ = p.best(dev_bytes)).dev) return TOPS_OK;
     }
-    // a new block, rounded up so that calls of about one size share it
+    // a new block, rounded up so that calls of about one size share it; one too
+    // large to be kept has no pinned part
     size_t n = 1u << 20;
     while (n < dev_bytes && n < kKeepBytes) n <<= 1;
     b_.bytes = std::max(n, dev_bytes);
     TOPS_HIP(hipMalloc(&b_.dev, b_.bytes));
-    if (host_bytes > kPinnedBytes || hipHostMalloc(&b_.host, kPinnedBytes, 0) != hipSuccess) {
+    if (b_.bytes <= kKeepBytes && host_bytes <= kPinnedBytes &&
+        hipHostMalloc(&b_.host, kPinnedBytes, 0) != hipSuccess) {
         b_.host = nullptr;
         (void)hipGetLastError();
     }
@@ -206,18 +233,12 @@ int CallScratch::take(size_t dev_bytes, size_t host_bytes)
 CallScratch::~CallScratch()
 {
     if (!b_.dev) return;
-    if (device_ >= 0 && device_ < kMaxDevices && b_.bytes <= kKeepBytes && b_.host && idle_) {
+    if (device_ >= 0 && b_.host && idle_) {
         ScratchPool& p = g_scratch[device_];
         std::lock_guard<std::mutex> lock(p.mu);
-        try {
-            if (p.idle.size() < kKeepBlocks) {
-                p.idle.push_back(b_);
-                return;
-            }
-        } catch (...) {
-        }
+        b_ = p.keep(b_);
     }
-    free_block(b_);   // (waits for the device)
+    free_block(b_);
 }
 
 int staged_upload(void* d_dst, const void* h_src, size_t bytes)

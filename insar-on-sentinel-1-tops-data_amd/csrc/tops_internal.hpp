@@ -157,8 +157,8 @@ int staged_download(void* h_dst, const void* d_src, size_t bytes);
 
 // Device scratch of one call and a small pinned host block that its last
 // kernel writes its result to (null: there is none, the result goes through
-// dev()).  Blocks of up to 8 MiB are kept for later calls, 4 idle ones per
-// device; a block is one call's alone from take() to the destructor.
+// dev()).  Blocks of up to 8 MiB are kept for later calls, the 4 largest idle
+// ones per device; a block is one call's alone from take() to the destructor.
 class CallScratch {
 public:
     struct Block {

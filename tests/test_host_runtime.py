@@ -136,6 +136,29 @@ def geocoreg(lines, pixels):
 """
 
 
+def test_kept_scratch_serves_the_larger_calls_too(run):
+    """Idle blocks of small calls give way to a larger one, a call takes the
+    smallest block that serves it, and one whose block is not kept takes no
+    pinned memory."""
+    run(CALLS + """
+S.stub_sync_ms(200)
+t = [threading.Thread(target=esd) for _ in range(4)]
+[x.start() for x in t]; [x.join() for x in t]
+S.stub_sync_ms(0)
+assert S.stub_host_blocks() == 4
+geocoreg(1500, 2200)                 # 5 MB of tile records
+made = count("hipMalloc")
+for _ in range(5):
+    geocoreg(1500, 2200)
+    esd()
+assert count("hipMalloc") == made, count("hipMalloc") - made
+pinned = count("hipHostMalloc")
+geocoreg(6000, 6000)                 # 50 MB
+assert count("hipHostMalloc") == pinned and S.stub_host_blocks() <= 4
+assert S.stub_bad() == 0
+""")
+
+
 def test_staging_pool_is_tried_again(run):
     """A pool that could not be made leaves a copy to the runtime, once."""
     run(CALLS + """
