@@ -228,6 +228,7 @@ void tops_ctx_destroy(tops_ctx* c)
     if (c->d_kaz_sh) (void)hipFree(c->d_kaz_sh);
     if (c->d_krgx) (void)hipFree(c->d_krgx);
     c->scratch.release();
+    release_idle_scratch();
     delete c;
 }
 

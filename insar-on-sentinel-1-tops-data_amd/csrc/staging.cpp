@@ -241,6 +241,14 @@ CallScratch::~CallScratch()
     free_block(b_);
 }
 
+void release_idle_scratch()
+{
+    for (ScratchPool& p : g_scratch) {
+        std::lock_guard<std::mutex> lock(p.mu);
+        for (CallScratch::Block b; (b = p.best(0)).dev;) free_block(b);
+    }
+}
+
 int staged_upload(void* d_dst, const void* h_src, size_t bytes)
 {
     if (bytes == 0) return TOPS_OK;

@@ -158,7 +158,8 @@ int staged_download(void* h_dst, const void* d_src, size_t bytes);
 // Device scratch of one call and a small pinned host block that its last
 // kernel writes its result to (null: there is none, the result goes through
 // dev()).  Blocks of up to 8 MiB are kept for later calls, the 4 largest idle
-// ones per device; a block is one call's alone from take() to the destructor.
+// ones per device, until a context is destroyed; a block is one call's alone
+// from take() to the destructor.
 class CallScratch {
 public:
     struct Block {
@@ -181,6 +182,9 @@ private:
     int device_ = -1;
     bool idle_ = false;
 };
+
+// gives the idle scratch blocks of all devices back
+void release_idle_scratch();
 
 // launchers (resample.hip)
 int launch_resample_fp64(tops_ctx* ctx, const ResampleParams& p, hipStream_t s);

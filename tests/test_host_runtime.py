@@ -159,6 +159,17 @@ assert S.stub_bad() == 0
 """)
 
 
+def test_kept_scratch_is_given_back(run):
+    """Destroying a context gives the idle scratch back."""
+    run(CALLS + """
+tables = S.stub_device_bytes()
+esd(); geocoreg(1500, 2200)
+assert S.stub_device_bytes() > tables and S.stub_host_blocks() > 0
+L.tops_ctx_destroy(ctx)
+assert S.stub_device_bytes() == 0 and S.stub_host_blocks() == 0 and S.stub_bad() == 0
+""")
+
+
 def test_staging_pool_is_tried_again(run):
     """A pool that could not be made leaves a copy to the runtime, once."""
     run(CALLS + """
