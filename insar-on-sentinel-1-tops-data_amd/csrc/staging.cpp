@@ -57,10 +57,12 @@ bool known(const void* h)
     return a.type != hipMemoryTypeUnregistered;
 }
 
-// The pool's buffers, made on first use.  A pool that cannot be made is tried again by the next call.
+// The pool's buffers, made on first use, and again after a device reset took
+// them.  A pool that cannot be made is tried again by the next call.
 bool pool_init(Pool& p)
 {
-    if (p.ready) return true;
+    if (p.ready && known(p.buf[0])) return true;
+    p.ready = false;
     p.s = nullptr;
     for (int k = 0; k < 2; k++) {
         p.buf[k] = nullptr;
@@ -214,7 +216,9 @@ int CallScratch::take(size_t dev_bytes, size_t host_bytes)
     if (device_ >= 0 && dev_bytes <= kKeepBytes && host_bytes <= kPinnedBytes) {
         ScratchPool& p = g_scratch[device_];
         std::lock_guard<std::mutex> lock(p.mu);
-        if ((b_ = p.best(dev_bytes)).dev) return TOPS_OK;
+        // (a block that the runtime no longer knows went with a device reset)
+        while ((b_ = p.best(dev_bytes)).dev)
+            if (known(b_.host)) return TOPS_OK;
     }
     // a new block, rounded up so that calls of about one size share it; one too
     // large to be kept has no pinned part
@@ -245,7 +249,8 @@ void release_idle_scratch()
 {
     for (ScratchPool& p : g_scratch) {
         std::lock_guard<std::mutex> lock(p.mu);
-        for (CallScratch::Block b; (b = p.best(0)).dev;) free_block(b);
+        for (CallScratch::Block b; (b = p.best(0)).dev;)
+            if (known(b.host)) free_block(b);
     }
 }
 

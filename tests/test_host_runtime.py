@@ -170,6 +170,23 @@ assert S.stub_device_bytes() == 0 and S.stub_host_blocks() == 0 and S.stub_bad()
 """)
 
 
+def test_calls_after_a_device_reset(run):
+    """Calls that hold nothing of the caller's take new scratch and staging
+    buffers when a reset of the device has taken the kept ones."""
+    run(CALLS + """
+big = np.zeros(3000 * 900 * 2, np.int16)     # a CInt16 raster of 10.8 MB
+coh = np.zeros(3000 * 900, np.float32)
+def drop_in():
+    d = L.ResampleFirstBurst(np.zeros(3000 * 900, np.complex64).ctypes.data, 900, 3000)
+    L.CoherenceEst_ESD(0, 0, 900, 3000, 4, 1, 10, 3, big.ctypes.data, d, N.ptr(coh, C.c_float))
+    assert L.tops_last_error() == 0
+esd(); drop_in()
+S.stub_reset()
+esd(); drop_in(); geocoreg(300, 300)
+assert S.stub_bad() == 0
+""")
+
+
 def test_staging_pool_is_tried_again(run):
     """A pool that could not be made leaves a copy to the runtime, once."""
     run(CALLS + """
