@@ -32,6 +32,7 @@ struct tops_plan {
     // -strip_rows lines (3 az x 10 rg window only)
     int strip_rows = 0;
     std::vector<ResampleParams> h_params;
+    bool even = true;          // every item's positions are (resample_even)
     std::vector<CohItem> h_coh;
     std::vector<int> coh_of;   // index into h_coh per item, or -1
     ResampleParams* d_params = nullptr;
@@ -149,6 +150,7 @@ int fill_params(tops_plan* p)
         r.out = it.out;
     }
     p->h_params = prm;
+    for (const ResampleParams& r : prm) p->even = p->even && resample_even(r);
     TOPS_HIP(hipMalloc(&p->d_params, sizeof(ResampleParams) * prm.size()));
     TOPS_HIP(hipMemcpy(p->d_params, prm.data(), sizeof(ResampleParams) * prm.size(),
                        hipMemcpyHostToDevice));
@@ -385,7 +387,8 @@ int enqueue(tops_plan* p, hipStream_t s, Marks* mk = nullptr)
             const int r0 = p->rs_off[g], nr = p->rs_off[g + 1] - r0;
             const int c0 = p->coh_off[g], nc = p->coh_off[g + 1] - c0;
             rc = marked(mk, s, kKindResample, [&] {
-                return launch_resample_batch(p->d_params, p->d_work_rs + r0, nr, p->rs_tall[g], s);
+                return launch_resample_batch(p->d_params, p->d_work_rs + r0, nr, p->rs_tall[g],
+                                             p->even, s);
             });
             if (rc || nc == 0) continue;
             TOPS_HIP(hipEventRecord(p->ev_grp[g], s));
@@ -404,7 +407,7 @@ int enqueue(tops_plan* p, hipStream_t s, Marks* mk = nullptr)
     // (groups in one launch: their tall and short strips alternate)
     const int n_tall = p->groups > 1 ? p->n_work_rs : p->rs_tall[0];
     rc = marked(mk, s, kKindResample, [&] {
-        return launch_resample_batch(p->d_params, p->d_work_rs, p->n_work_rs, n_tall, s);
+        return launch_resample_batch(p->d_params, p->d_work_rs, p->n_work_rs, n_tall, p->even, s);
     });
     if (rc) return rc;
     if (p->coh_batched)

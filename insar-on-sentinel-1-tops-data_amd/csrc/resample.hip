@@ -141,9 +141,9 @@ int launch_resample_fp64(tops_ctx* ctx, const ResampleParams& p, hipStream_t s)
 //     writes it to LDS;
 //   * each output then needs only its own 12 range taps over U, and its
 //     phase.
-// Outputs whose key or window the shared pass cannot serve (a key beyond the
-// window's reach, or a range window outside the strip's 64 columns) are
-// computed by interior_direct.
+// Outputs that the shared pass cannot serve (a range window outside the strip's
+// 64 columns, a key out of the window's reach at all its positions) are computed
+// by interior_direct.
 //
 // Why groups: one row at a time is a chain of dependent latencies (position
 // -> keys -> tap loads -> LDS exchange -> range sums) and of scalar loads that
@@ -296,19 +296,20 @@ __device__ __forceinline__ int trunc_i32(double v)
     return r;
 }
 
-// the smallest value of the wave (uniform; values 0 .. INT_MAX): the largest
-// complement, whose identity is the 0 that a lane without a source reads
-__device__ __forceinline__ int wave_min(int v)
+// the largest value of the wave (uniform; values 0 .. INT_MAX): 0 is what a
+// lane without a source reads
+__device__ __forceinline__ int wave_max(int v)
 {
-    unsigned u = (unsigned)v ^ 0x7fffffffu;
+    unsigned u = (unsigned)v;
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x111, 0xf, 0xf, true));    // row_shr:1
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x112, 0xf, 0xf, true));    // row_shr:2
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x114, 0xf, 0xf, true));    // row_shr:4
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x118, 0xf, 0xf, true));    // row_shr:8
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x142, 0xa, 0xf, false));   // row_bcast:15
     u = max(u, (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, 0x143, 0xc, 0xf, false));   // row_bcast:31
-    return __builtin_amdgcn_readlane((int)u, 63) ^ 0x7fffffff;
+    return __builtin_amdgcn_readlane((int)u, 63);
 }
+__device__ __forceinline__ int wave_min(int v) { return wave_max(v ^ INT_MAX) ^ INT_MAX; }
 
 // value k[lane & 3] of four uniform values
 __device__ __forceinline__ int by_row(int k0, int k1, int k2, int k3, bool b0, bool b1)
@@ -319,14 +320,22 @@ __device__ __forceinline__ int by_row(int k0, int k1, int k2, int k3, bool b0, b
 
 // Output rows r0 .. r1-1 of the strip whose lane 0 is output column c0 and
 // slave column ucol0, in groups of 4.  kSmooth: the fitted phase; otherwise
-// FP64 phases per column.
-template <bool kSmooth>
+// FP64 phases per column.  kEven: the slave line advances by about one a row
+// and hardly along it, so that the window slides by 4 lines from group to group
+// and reaches all of a group's keys; the few outputs it does not reach are left
+// to the direct path.  Otherwise it slides by any number of lines, and to
+// further positions for keys it does not reach: that handling costs the even
+// rows 4 to 6 % (1500 x 21000: 232 us and 246).
+template <bool kSmooth, bool kEven>
 __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r0, int r1,
                                           int ucol0, ColumnWalker& w, WalkLds& sm)
 {
     constexpr int G = WK_GROUP;
     constexpr int S = kSmooth ? WK_SLOTS : 1;   // azimuth keys per row and round
-    constexpr int kReach = kAzShifts - 1;       // lines past the group's first a key may start at
+    constexpr int kReach = kAzShifts - 1;       // lines past the window's first a key may start at
+    constexpr int kWaveShr1 = 0x138;            // DPP: the value of the lane to the left
+    constexpr int kMaxSlide = 20;               // lines the window slides rather than start anew
+    constexpr int kMaxMoves = 16;               // window positions after a group's first
     static_assert(32 % G == 0, "the row table is refreshed between groups");
     const int lane = threadIdx.x;
     const int c = c0 + lane;
@@ -346,7 +355,8 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
     int wbase = INT_MIN;           // absolute slave line held in win[0]
     bool late = false;             // outputs are marked for the direct path (uniform)
     // A group takes one round of up to S keys per row, or further rounds
-    // (again) where a row segment holds more; a round keeps the positions.
+    // (again) where a row segment holds more, or its keys are further apart than
+    // the window reaches; a round keeps the positions.
     // key: line * 2048 + LUT row of an output the shared pass may serve
     // (INT_MAX: none); fxo: byte offset of its range LUT row; xt: its first
     // tap's lane, from u0; heads: the lanes that list the row's keys not yet
@@ -354,6 +364,8 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
     int key[G], fxo[G], xt[G], line0 = 0;
     unsigned long long heads[G], need[G];
     bool again = false;
+    bool place = true;   // !kEven: the window is to be placed
+    int moves = 0;       // and its positions since the group's first
     for (int r = r0; r < r1;) {
         if (!again) {
             // ---- row-uniform position terms, 32 rows at a time (one per lane)
@@ -410,7 +422,6 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             // (interior rows of a slave box checked at launch).
 #pragma unroll
             for (int i = 0; i < G; i++) {
-                constexpr int kWaveShr1 = 0x138;   // DPP: the value of the lane to the left
                 const int kleft = __builtin_amdgcn_update_dpp(~key[i], key[i], kWaveShr1, 0xf, 0xf,
                                                               false);
                 heads[i] = __builtin_amdgcn_ballot_w64(key[i] != INT_MAX) &
@@ -420,13 +431,37 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             line0 = wave_min(min(min(key[0], key[1]), min(key[2], key[3]))) >> 11;
         }
         if (line0 != INT_MAX >> 11) {
+            int wline = line0;   // the first line a key may start at
+            int slide = 0, steps = 0;
+            if constexpr (!kEven) {
+                // the window is to hold lines line0-5 onwards: it slides by
+                // fours (-1: starts anew), and by single lines too where that
+                // reaches further keys
+                if (place) {
+                    slide = wbase == INT_MIN ? -1 : line0 - kHalf - wbase;
+                    if (slide >= 0 && slide <= kMaxSlide) {
+                        int last = 0;
+#pragma unroll
+                        for (int i = 0; i < G; i++)
+                            last = max(last, key[i] == INT_MAX ? 0 : key[i]);
+                        if ((wave_max(last) >> 11) - line0 + (slide & 3) > kReach) steps = slide & 3;
+                        wbase = line0 - kHalf - (slide & 3) + steps;
+                        slide >>= 2;
+                    } else {
+                        slide = -1;
+                        wbase = line0 - kHalf;
+                    }
+                    place = false;
+                }
+                wline = wbase + kHalf;
+            }
             // ---- this round's keys (uniform; -1: none).  A key whose
-            // lines lie beyond the window's reach is left to the direct path.
-            // A key that reappears further along the row is served by its
-            // first slot.
+            // lines lie beyond the window's reach is left to its next position
+            // (kEven: to the direct path).  A key that reappears further along the
+            // row is served by its first slot.
             // (no head left reads lane 63, which owns no output)
             int kq[G][S];
-            const int lim = (line0 + kReach) << 11 | (kLutRows - 1);
+            const int lim = (wline + kReach) << 11 | (kLutRows - 1);
 #pragma unroll
             for (int i = 0; i < G; i++) {
 #pragma unroll
@@ -449,8 +484,8 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
 #pragma unroll
             for (int s = 0; s < S; s++) {
                 kr[s] = by_row(kq[0][s], kq[1][s], kq[2][s], kq[3][s], b0, b1);
-                if (kr[s] < 0) kr[s] = line0 << 11;
-                wt[s] = p.kaz_sh[((((kr[s] >> 11) - line0) * kLutRows + (kr[s] & (kLutRows - 1)))
+                if (kr[s] < 0) kr[s] = wline << 11;
+                wt[s] = p.kaz_sh[((((kr[s] >> 11) - wline) * kLutRows + (kr[s] & (kLutRows - 1)))
                                   * kAzShiftTaps) + (lane >> 2)];
             }
             float4 tap[2][4];
@@ -462,7 +497,20 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             };
             if (lane < WK_OUT) load_range(0);
             __builtin_amdgcn_sched_barrier(0);
-            if (!again) {
+            if constexpr (!kEven) {
+                if (__builtin_expect(slide < 0, 0)) {
+                    w.anchor(p, wbase, sm.abc[0][lane], sm.abc[1][lane], sm.abc[2][lane]);
+                    int raw[WK_WIN];
+#pragma unroll
+                    for (int k = 0; k < WK_WIN; k++) raw[k] = w.fetch(p, wbase + k);
+#pragma unroll
+                    for (int k = 0; k < WK_WIN; k++) win[k] = win_pack(w.deramp(raw[k]));
+                    w.prefetch(p);
+                } else {
+                    for (; slide > 0; slide--) slide4(win, w, p);
+                    for (; steps > 0; steps--) slide1(win, w, p);
+                }
+            } else if (!again) {
                 // the window holds lines wbase .. wbase+15; lines line0-5
                 // onwards are wanted.  It slides by 4 lines, which is what 4
                 // output rows advance by; positions that advance otherwise (a
@@ -548,6 +596,7 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
                 const bool s1 = S == 2 && key[i] == kq[i][S - 1];
                 if (i + 1 < G) load_range(i + 1);   // the next row's taps
                 __builtin_amdgcn_sched_barrier(0);
+                if (!kEven && mine[i] == 0ull) continue;   // (uniform)
                 const float4 k0 = tap[i & 1][0], k1 = tap[i & 1][1], k2 = tap[i & 1][2];
                 const float4 km = tap[i & 1][3];
                 const float kp[kTaps] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y,
@@ -603,12 +652,35 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             again = (heads[0] | heads[1] | heads[2] | heads[3]) != 0ull;
         }
         if (__builtin_expect(again, 0)) continue;
+        if constexpr (!kEven) place = true;
 
         // ---- the outputs no round served: outside the box (0), in its edge
         // band (the sample itself), or marked for the direct path.  The four
         // rows together: edge strips would otherwise wait for one load a row
         // and end long after the others
         if (__builtin_expect((need[0] | need[1] | need[2] | need[3]) != 0ull, 0)) {
+            if constexpr (!kEven) {
+                // keys beyond the window's reach first: rounds at its next position
+                unsigned long long far[G];
+#pragma unroll
+                for (int i = 0; i < G; i++)
+                    far[i] = need[i] & __builtin_amdgcn_ballot_w64(key[i] != INT_MAX);
+                if ((far[0] | far[1] | far[2] | far[3]) != 0ull && moves < kMaxMoves) {
+                    int first = INT_MAX;
+#pragma unroll
+                    for (int i = 0; i < G; i++) {
+                        first = min(first,
+                                    __builtin_amdgcn_inverse_ballot_w64(far[i]) ? key[i] : INT_MAX);
+                        const int kleft = __builtin_amdgcn_update_dpp(~key[i], key[i], kWaveShr1,
+                                                                      0xf, 0xf, false);
+                        heads[i] = far[i] & __builtin_amdgcn_ballot_w64(kleft != key[i]);
+                    }
+                    line0 = wave_min(first) >> 11;
+                    again = place = true;
+                    moves++;
+                    continue;
+                }
+            }
             int reg[G];
             tops_ci16 v[G];
 #pragma unroll
@@ -629,6 +701,7 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
                     stream_store_float2(p.out + (size_t)(r + i) * p.m_pixels + (unsigned)c, o.x, o.y);
             }
         }
+        if constexpr (!kEven) moves = 0;
         r += G;
     }
 
@@ -653,6 +726,7 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
 // One strip of one burst: output columns sx*WK_OUT .. +WK_OUT-1, output rows
 // r0 .. r1-1 of the master box.  p may live in global memory (batched
 // launches): its fields are wave-uniform.
+template <bool kEven>
 __device__ __forceinline__ void resample_strip(const ResampleParams& p, int sx, int r0, int r1,
                                                WalkLds& sm)
 {
@@ -704,9 +778,9 @@ __device__ __forceinline__ void resample_strip(const ResampleParams& p, int sx, 
         phasor(2.0 * cc, w.qr, w.qi);
     }
     if (fit_phase(p, sm, ucol0))
-        walk_rows<true>(p, c0, r0, r1, ucol0, w, sm);
+        walk_rows<true, kEven>(p, c0, r0, r1, ucol0, w, sm);
     else
-        walk_rows<false>(p, c0, r0, r1, ucol0, w, sm);
+        walk_rows<false, kEven>(p, c0, r0, r1, ucol0, w, sm);
 }
 
 // The strip of workgroup b of n: the first n_tall strips, then the others, each
@@ -720,8 +794,9 @@ __device__ __forceinline__ int strip_remap(int b, int n_tall, int n)
 // Batched form: one workgroup per entry of a strip table covering many
 // bursts (work[i] = {burst, strip x, first row, rows}; the first n_tall entries
 // are the tall strips).
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWalkWavesPerSimd))) resample_batch_kernel(const ResampleParams* items,
-                                                            const int4* work, int n_tall)
+template <bool kEven>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWalkWavesPerSimd)))
+resample_batch_kernel(const ResampleParams* items, const int4* work, int n_tall)
 {
     __shared__ WalkLds sm;
     // the table and the parameter blocks are read-only and read with
@@ -732,7 +807,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWalkWa
     const CInt* w = (const CInt*)work + 4 * strip_remap((int)blockIdx.x, n_tall, (int)gridDim.x);
     const int item = w[0], sx = w[1], r0 = w[2], rows = w[3];
     CParams* it = (CParams*)items + item;
-    resample_strip(*(const ResampleParams*)it, sx, r0, min(r0 + rows, it->m_lines), sm);
+    resample_strip<kEven>(*(const ResampleParams*)it, sx, r0, min(r0 + rows, it->m_lines), sm);
 }
 
 // Row ranges of up to kItems bursts in one launch, the parameter blocks in the
@@ -748,7 +823,7 @@ struct ResampleSet {
 };
 static_assert(sizeof(ResampleSet<kResampleSetItems>) <= 4096, "kernel argument segment");
 
-template <int kItems>
+template <int kItems, bool kEven>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWalkWavesPerSimd)))
 resample_fast_kernel(ResampleSet<kItems> set)
 {
@@ -768,7 +843,7 @@ resample_fast_kernel(ResampleSet<kItems> set)
     const int sx = t / ny, sy = t - sx * ny;
     const int r0 = k->seg[i].row0 + sy * h;
     const int r1 = min(r0 + h, k->seg[i].row0 + rows);
-    resample_strip(*(const ResampleParams*)&k->item[k->seg[i].item], sx, r0, r1, sm);
+    resample_strip<kEven>(*(const ResampleParams*)&k->item[k->seg[i].item], sx, r0, r1, sm);
 }
 
 int resample_strip_columns(int m_pixels) { return (m_pixels + WK_OUT - 1) / WK_OUT; }
@@ -858,6 +933,30 @@ static StripHeights resample_heights(const int* lines, const int* pixels, int n)
     return resample_heights_of(h - 3 * WK_GROUP, lines, pixels, n);
 }
 
+// Whether the walker's form for even positions serves an item: over the whole
+// box the slave line advances by 1 within 1/32 a row, so that the window starts
+// anew at most every 8 groups, and 4 rows of a strip spread over at most 4
+// lines.  Both slopes are linear: their extremes are at the box's corners.  A
+// false comparison, as of NaN, takes the other form, which serves everything.
+// (1500 x 12000, this form against the other, us: 1 line a row 160 / 168, 0.98
+// 150 / 155, 1.02 148 / 149, 0.95 154 / 151, 0.9 159 / 151, 0.8 174 / 153, 0.5 191
+// / 148, 2 2560 / 222; lines a column 0.018 2260 / 2444, 0.025 3200 / 2520.  The
+// walker of one row at a time: 200 at 1, 177 at 0.5, 192 at 2 lines a row.)
+bool resample_even(const ResampleParams& p)
+{
+    const double per_row = 4.0 / (p.mb[3] - p.mb[2]), per_col = 4.0 / (p.mb[1] - p.mb[0]);
+    for (int k = 0; k < 4; k++) {
+        const double ln = k & 1 ? 2.0 : -2.0, pn = k & 2 ? 2.0 : -2.0;
+        const double* c = p.cpm_az;
+        const double rate = (c[1] + 2.0 * c[3] * ln + c[4] * pn) * per_row;
+        const double shear = (c[2] + c[4] * ln + 2.0 * c[5] * pn) * per_col;
+        if (!(std::fabs(rate - 1.0) <= 1.0 / 32 &&
+              (WK_GROUP - 1) * rate + WK_OUT * std::fabs(shear) <= kAzShifts - 1))
+            return false;
+    }
+    return true;
+}
+
 static int check_slave_bytes(const ResampleParams& p)
 {
     if ((long long)p.s_lines * p.s_pixels * 4 > kMaxSlaveBytes)
@@ -892,7 +991,12 @@ static int launch_set(const ResampleParams* items, int base, const int (*range)[
         add(range[i][0] - base, range[i][1] + range[i][2] - n, n, sh.low);
     }
     if (strips == 0) return TOPS_OK;
-    hipLaunchKernelGGL(resample_fast_kernel<kItems>, dim3(strips), dim3(64), 0, s, set);
+    bool even = true;
+    for (int i = i0; i < i1; i++) even = even && resample_even(items[range[i][0]]);
+    if (even)
+        hipLaunchKernelGGL((resample_fast_kernel<kItems, true>), dim3(strips), dim3(64), 0, s, set);
+    else
+        hipLaunchKernelGGL((resample_fast_kernel<kItems, false>), dim3(strips), dim3(64), 0, s, set);
     TOPS_HIP(hipGetLastError());
     return TOPS_OK;
 }
@@ -937,11 +1041,15 @@ int launch_resample_set(const ResampleParams* items, int n_items, const int (*ra
 }
 
 int launch_resample_batch(const ResampleParams* d_items, const int4* d_work, int n_work,
-                          int n_tall, hipStream_t s)
+                          int n_tall, bool even, hipStream_t s)
 {
     if (n_work <= 0) return TOPS_OK;
-    hipLaunchKernelGGL(resample_batch_kernel, dim3(n_work), dim3(64), 0, s, d_items, d_work,
-                       n_tall);
+    if (even)
+        hipLaunchKernelGGL(resample_batch_kernel<true>, dim3(n_work), dim3(64), 0, s, d_items,
+                           d_work, n_tall);
+    else
+        hipLaunchKernelGGL(resample_batch_kernel<false>, dim3(n_work), dim3(64), 0, s, d_items,
+                           d_work, n_tall);
     TOPS_HIP(hipGetLastError());
     return TOPS_OK;
 }

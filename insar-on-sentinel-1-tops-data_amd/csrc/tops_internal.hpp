@@ -194,9 +194,11 @@ int launch_resample_fast(const ResampleParams& p, hipStream_t s, int strip_rows 
 constexpr int kResampleSetItems = 11;
 int launch_resample_set(const ResampleParams* items, int n_items, const int (*range)[3],
                         int n_range, hipStream_t s);
-// strips {item, strip column, first row, rows}, the first n_tall the tall ones
+bool resample_even(const ResampleParams& p);
+// strips {item, strip column, first row, rows}, the first n_tall the tall ones;
+// even: resample_even of every item
 int launch_resample_batch(const ResampleParams* d_items, const int4* d_work, int n_work,
-                          int n_tall, hipStream_t s);
+                          int n_tall, bool even, hipStream_t s);
 int resample_strip_columns(int m_pixels);
 // heights of a launch's strips: `tall`, and `low` for the last low_rows() rows
 // of each row range

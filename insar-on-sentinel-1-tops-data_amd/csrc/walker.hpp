@@ -293,6 +293,21 @@ __device__ __forceinline__ void slide4(Win (&win)[WK_WIN], ColumnWalker& w,
     for (int k = 0; k < 4; k++) win[WK_WIN - 4 + k] = win_pack(w.deramp(v[k]));
 }
 
+// Slide a window by one row (rare: the pending lines move up, which waits for
+// them)
+template <typename Win>
+__device__ __forceinline__ void slide1(Win (&win)[WK_WIN], ColumnWalker& w,
+                                       const ResampleParams& p)
+{
+    const int raw = w.pend[0];
+#pragma unroll
+    for (int k = 0; k < 3; k++) w.pend[k] = w.pend[k + 1];
+    w.pend[3] = w.fetch(p, w.ynext + 4);
+#pragma unroll
+    for (int k = 0; k < WK_WIN - 1; k++) win[k] = win[k + 1];
+    win[WK_WIN - 1] = win_pack(w.deramp(raw));
+}
+
 // read-only tables addressed with wave-uniform indices
 typedef __attribute__((address_space(4))) const float CFloat;
 typedef __attribute__((address_space(4))) const double CDouble;
