@@ -184,19 +184,27 @@ tops_ctx* tops_ctx_create(const float* kernel_az, const float* kernel_rg, int np
     std::vector<float> rx((size_t)kLutRows * kKrgxRow);
     c->krg_unit = 1;
     for (int r = 0; r < kLutRows; r++) {
-        double e0 = -1.0, m1 = 0, m2 = 0;
+        double e0 = -1.0, m1 = 0, v = 0, c3 = 0;
         float* q = &rx[(size_t)r * kKrgxRow];
         for (int j = 0; j < kTaps; j++) {
-            const double k = (double)kernel_rg[r * kTaps + j], u = (double)(j - kHalf);
+            const double k = (double)kernel_rg[r * kTaps + j];
             e0 += k;
-            m1 += k * u;
-            m2 += k * u * u;
+            m1 += k * (j - kHalf);
             q[j] = kernel_rg[r * kTaps + j];
         }
-        if (!(fabs(e0) <= kUnitSum)) c->krg_unit = 0;
-        memcpy(q + kTaps, &m1, sizeof(m1));
+        const double mu = m1 / (1.0 + e0);
+        for (int j = 0; j < kTaps; j++) {
+            const double k = (double)q[j], u = (double)(j - kHalf) - mu;
+            v += k * u * u;
+            c3 += k * u * u * u;
+        }
+        // (a false comparison, as of a NaN, leaves the row to the general form)
+        if (!(fabs(e0) <= kUnitSum && fabs(e0 - (double)(float)e0) <= kUnitSumRounding &&
+              fabs(v) <= 1.0 && fabs(c3) <= 1.0))
+            c->krg_unit = 0;
+        memcpy(q + kTaps, &mu, sizeof(mu));
         q[kTaps + 2] = (float)e0;
-        q[kTaps + 3] = (float)m2;
+        q[kTaps + 3] = (float)v;
     }
     hipError_t e = hipMalloc(&c->d_kaz, lut);
     if (e == hipSuccess) e = hipMalloc(&c->d_krg, lut);

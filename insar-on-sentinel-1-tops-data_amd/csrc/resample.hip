@@ -152,26 +152,31 @@ int launch_resample_fp64(tops_ctx* ctx, const ResampleParams& p, hipStream_t s)
 //
 // What bounds it: vector issue, about three quarters of the time (one IW
 // burst, 1500 x 21000, moves 0.38 GB: 60 us of memory time).  Measured there,
-// on one GPU: 232 us, against 292-335 for the row-at-a-time walker with scalar
+// on one GPU: 233 us, against 292-335 for the row-at-a-time walker with scalar
 // tap loads and 12 FP64 phases an output (265-273 before the launch ended in low
-// strips and the azimuth shift was a scalar load).  3 waves per SIMD (155
+// strips and the azimuth shift was a scalar load).  3 waves per SIMD (161
 // VGPRs): 2 take 238 us; at 4 the registers spill into the row loop (266); at 6
 // to 9, with a wave pair sharing a strip, 307 to 608 at the 265 us stage.
 //
 // The phase.  Phi is the 12 x 12 tap sum of phi(y, x) = a(x) + b(x) y +
-// c(x) y^2.  Over a strip's 64 columns a, b and c are quadratics of the
-// column to far below FP64's use of them (they come from quadratic Doppler
-// centroid and FM rate polynomials), so the range sum collapses to the tap
-// moments of the output's LUT row as the azimuth sum does (walk kSmooth):
-// 9 FP64 operations an output instead of 24 and 12 LDS reads.  The strip
-// checks its own arrays: every column's residual from the quadratic through
-// three of its columns must stay below kSmoothTol (half an ulp of an FP32
-// sample of magnitude 1) on every slave line; otherwise it sums the 12
-// columns' FP64 phases.
+// c(x) y^2.  Over a strip's 64 columns a, b and c are cubics of the column to
+// their own FP64 rounding (they come from quadratic Doppler centroid and FM rate
+// polynomials), so the range sum collapses to the tap moments of the output's
+// LUT row as the azimuth sum does (walk kSmooth): 10 FP64 operations an output
+// instead of 24 and 12 LDS reads (a quadratic fit leaves out up to 1e-8 rad at
+// 2000 columns a burst and 5e-7 at 320; it took 231 us here, and bursts below 700
+// columns the column sums: 1500 x 500 60 us, now 35).  The strip checks its own
+// arrays: on every
+// slave line every column's residual from the cubic through four of its columns
+// must stay below a bound of the order of the FP64 sum's rounding (fit_phase);
+// otherwise it sums the 12 columns' FP64 phases.
 
 constexpr int WK_GROUP = 4;           // output rows per group (one matrix-instruction block)
 constexpr int WK_SLOTS = 2;           // azimuth keys per row and round
-constexpr double kSmoothTol = 0x1p-25;   // rad
+// What the fitted phase may leave out: 2^-32 rad and 2^-47 of the size of the
+// phase's terms, a few roundings of the FP64 sum it takes the place of, and
+// never more than half an ulp of an FP32 sample of magnitude 1
+constexpr double kSmoothTol = 0x1p-32, kSmoothRel = 0x1p-47, kSmoothMax = 0x1p-25;
 
 struct WalkLds {
     // azimuth sums U: [row * WK_SLOTS + slot][column]; the general form holds
@@ -180,9 +185,9 @@ struct WalkLds {
     float2 u[WK_GROUP * WK_SLOTS][64];
     double rowt[32][6];         // row-uniform position terms of 32 rows
     double pos[5][64];          // per lane: Pn, c2 Pn and c5 Pn Pn of both polynomials
-    double ph[WK_GROUP][WK_SLOTS][4];  // smooth: the row's phase per key as a quadratic of the column
+    double ph[WK_GROUP][WK_SLOTS][6];  // smooth: the row's phase per key as a cubic of the column
     double abc[3][64];          // per lane: the column's phase coefficients a, b, c
-    double fit[9];              // smooth: a(x), b(x), c(x) in revolutions, quadratics of t, the
+    double fit[3][4];           // smooth: a(x), b(x), c(x) in revolutions, cubics of t, the
                                 // column less that of the 6th tap of the first servable window
 };
 static_assert(sizeof(WalkLds) <= 10240, "16 workgroups per CU");
@@ -192,59 +197,64 @@ __device__ __forceinline__ double lane_value(double v, int lane)
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                             __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
-// The quadratic of lane - t1 through the values of lanes t0 < t1 < t2
-// (uniform; h = t1 - t0 and the reciprocals of the spacings), in
-// revolutions, and this lane's residual from it in radians.
-__device__ __forceinline__ double fit_quadratic(double v, int t0, int t1, int t2, double t,
-                                                double h, double rh01, double rh12, double rh02,
-                                                double q[3])
-{
-    const double f0 = lane_value(v, t0), f1 = lane_value(v, t1), f2 = lane_value(v, t2);
-    const double d01 = (f1 - f0) * rh01, d12 = (f2 - f1) * rh12;
-    const double dd = (d12 - d01) * rh02;
-    const double s = fma(dd, h, d01);
-    q[0] = f1 * kInvTwoPi;
-    q[1] = s * kInvTwoPi;
-    q[2] = dd * kInvTwoPi;
-    return v - fma(t, fma(t, dd, s), f1);
-}
-
-// Fits the strip's phase coefficients into sm.fit (false: not smooth enough
-// on the slave box's lines, which hold every interior output's).
+// Fits the strip's phase coefficients into sm.fit, each the cubic through its
+// values at four columns near the Chebyshev places (false: not smooth enough on
+// the slave box's lines, which hold every interior output's).
 __device__ __forceinline__ bool fit_phase(const ResampleParams& p, WalkLds& sm, int ucol0)
 {
     const int lane = threadIdx.x;
     const int l0 = max(0, p.sb[0] - ucol0), l1 = min(63, p.sb[1] - ucol0);
     const int span = l1 - l0;
-    const int tc = (l0 + l1) >> 1;
-    if (span < 2 || !p.krg_unit) return false;
-    const int edge = span >> 4;
-    // the residual phase is a quadratic of the line: its values at the ends
-    // and the middle of the box bound it within a factor 1.25 in between
+    if (span < 3 || !p.krg_unit) return false;
+    const int out = (span * 5 + 64) >> 7, in = (span * 79 + 128) >> 8;
+    const int t0 = l0 + out, t1 = l0 + in, t2 = l1 - in, t3 = l1 - out;
+    const double x0 = (double)(lane - t0), x1 = (double)(lane - t1), x2 = (double)(lane - t2);
+    // the column of t = 0, from the places
+    const double a0 = (double)(l0 + kHalf - t0), a1 = (double)(l0 + kHalf - t1);
+    const double a2 = (double)(l0 + kHalf - t2);
+    const double ro = 1.0 / (double)(t1 - t0), ri = 1.0 / (double)(t2 - t1);
+    const double r2 = 1.0 / (double)(t2 - t0), r3 = 1.0 / (double)(t3 - t0);
+    // What the fit leaves out of the phase is a quadratic of the line: its values
+    // at the ends and the middle of the box bound it within a factor 1.25 in
+    // between.  It is this lane's residual, the third moment of the taps (below
+    // 1) times the cubic's leading coefficient, and the rounding of their second.
     const double y0 = (double)p.sb[2] - (double)p.first_line;
-    const double y2 = (double)p.sb[3] - (double)p.first_line, y1 = 0.5 * (y0 + y2);
-    double e0 = 0.0, e1 = 0.0, e2 = 0.0, s0 = 1.0, s1 = 1.0, s2 = 1.0;
-    const int t0 = l0 + edge, t2 = l1 - edge;
-    const double h = (double)(tc - t0), h2 = (double)(t2 - tc), t = (double)(lane - tc);
-    const double org = (double)(l0 + kHalf - tc);   // the column of t = 0
-    const double rh01 = 1.0 / h, rh12 = 1.0 / h2, rh02 = 1.0 / (h + h2);
+    const double y2 = (double)p.sb[3] - (double)p.first_line;
+    const double y[3] = {y0, 0.5 * (y0 + y2), y2}, ym = fmax(fabs(y0), fabs(y2));
+    double e[3] = {}, third[3] = {}, second[3] = {}, size = 0.0, yk[3] = {1.0, 1.0, 1.0}, ymk = 1.0;
 #pragma unroll 1
     for (int k = 0; k < 3; k++) {
-        double q[3];
-        const double res = fit_quadratic(sm.abc[k][lane], t0, tc, t2, t, h, rh01, rh12, rh02, q);
-        e0 = fma(s0, res, e0);
-        e1 = fma(s1, res, e1);
-        e2 = fma(s2, res, e2);
-        s0 *= y0;
-        s1 *= y1;
-        s2 *= y2;
-        sm.fit[3 * k] = fma(org, fma(org, q[2], q[1]), q[0]);
-        sm.fit[3 * k + 1] = fma(2.0 * org, q[2], q[1]);
-        sm.fit[3 * k + 2] = q[2];
+        const double v = sm.abc[k][lane];
+        const double f0 = lane_value(v, t0), f1 = lane_value(v, t1), f2 = lane_value(v, t2);
+        const double d01 = (f1 - f0) * ro, d12 = (f2 - f1) * ri, d23 = (lane_value(v, t3) - f2) * ro;
+        const double d02 = (d12 - d01) * r2, d3 = ((d23 - d12) * r2 - d02) * r3;
+        // f0 + (x - t0)(d01 + (x - t1)(d02 + (x - t2) d3)) about t = 0
+        const double u = fma(a2, d3, d02), w = fma(a1, d3, u), c2 = fma(a0, d3, w);
+        const double z = fma(a1, u, d01);
+        sm.fit[k][0] = fma(a0, z, f0) * kInvTwoPi;
+        sm.fit[k][1] = fma(a0, w, z) * kInvTwoPi;
+        sm.fit[k][2] = c2 * kInvTwoPi;
+        sm.fit[k][3] = d3 * kInvTwoPi;
+        const double res = v - fma(x0, fma(x1, fma(x2, d3, d02), d01), f0);
+        size = fma(ymk, fabs(v), size);
+        ymk *= ym;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            e[j] = fma(yk[j], res, e[j]);
+            third[j] = fma(yk[j], d3, third[j]);
+            second[j] = fma(yk[j], c2, second[j]);
+            yk[j] *= y[j];
+        }
+    }
+    double r = 0.0, nan = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        r = fmax(r, fabs(e[j]) + fabs(third[j]) + 0x1p-24 * fabs(second[j]));
+        nan += 0.0 * (e[j] + third[j] + second[j]);
     }
     // (fmax drops a NaN: the sum keeps it, and a NaN fails the comparison)
-    const double r = 1.25 * fmax(fabs(e0), fmax(fabs(e1), fabs(e2))) + 0.0 * (e0 + e1 + e2);
-    return __ballot(lane >= l0 && lane <= l1 && !(r <= kSmoothTol)) == 0ull;
+    const double tol = fmin(kSmoothTol + kSmoothRel * size, kSmoothMax);
+    return __ballot(lane >= l0 && lane <= l1 && !(1.25 * r + nan <= tol)) == 0ull;
 }
 
 // The mark of an interior output left to the direct path, in its place in the
@@ -560,21 +570,19 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             }
             if (kSmooth) {
                 // lane 4 s + i: the phase of row i and slot s, P0 + P1 t + P2
-                // t^2 over t = column of the 6th tap less the one of xt = 0,
-                // in revolutions
+                // t^2 + P3 t^3 over t = column of the 6th tap less the one of
+                // xt = 0, in revolutions, and 3 P3
                 const int kl = lane < G ? kr[0] : kr[S - 1];
                 if (lane < G * S) {
                     const double4 m = reinterpret_cast<const double4*>(p.mom)[kl & (kLutRows - 1)];
-                    const double* f = sm.fit;
                     const double y0 = (double)((kl >> 11) - p.first_line);
                     const double n1 = fma(y0, m.x, m.y);
                     const double n2 = y0 * y0 * m.x + 2.0 * y0 * m.y + m.z;
                     double* q = sm.ph[lane & 3][lane >> 2];
-                    q[0] = fma(m.x, f[0], fma(n1, f[3], n2 * f[6]));
-                    q[1] = fma(m.x, f[1], fma(n1, f[4], n2 * f[7]));
-                    const double q2 = fma(m.x, f[2], fma(n1, f[5], n2 * f[8]));
-                    q[2] = q2;
-                    q[3] = 2.0 * q2;
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        q[k] = fma(m.x, sm.fit[0][k], fma(n1, sm.fit[1][k], n2 * sm.fit[2][k]));
+                    q[4] = 3.0 * q[3];
                 }
             }
             __syncthreads();
@@ -620,16 +628,16 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
                 }
                 double ph;
                 if (kSmooth) {
-                    // sum_k kp (P0 + P1 t_k + P2 t_k^2), t_k = t + k - 5: with
-                    // the LUT row's moments 1 + e0, m1, m2 this is
-                    // (1 + e0) Q(t) + m1 Q'(t) + m2 P2
+                    // sum_k kp P(t + k - 5): with the LUT row's sum 1 + e0, mean
+                    // offset mu and second moment about it, v, this is
+                    // (1 + e0) P(x) + v P''(x) / 2 at x = t + mu (the third
+                    // moment is left out: fit_phase)
                     const double* q = sm.ph[i][s1 ? 1 : 0];
-                    const double P0 = q[0], P1 = q[1], P2 = q[2], P2x2 = q[3];
-                    const double t = (double)xt[i];
-                    const double m1 = __hiloint2double(__float_as_int(km.y), __float_as_int(km.x));
-                    const double Q = fma(t, fma(t, P2, P1), P0);
-                    ph = fma(m1, fma(t, P2x2, P1),
-                             fma((double)km.w, P2, fma((double)km.z, Q, Q)));
+                    const double P0 = q[0], P1 = q[1], P2 = q[2], P3 = q[3], P3x3 = q[4];
+                    const double x = (double)xt[i] +
+                                     __hiloint2double(__float_as_int(km.y), __float_as_int(km.x));
+                    const double Q = fma(x, fma(x, fma(x, P3, P2), P1), P0);
+                    ph = fma((double)km.w, fma(x, P3x3, P2), fma((double)km.z, Q, Q));
                 } else {
                     const double* pl = reinterpret_cast<const double*>(u0) + (WK_GROUP + i) * 64 + xt[i];
                     ph = 0.0;

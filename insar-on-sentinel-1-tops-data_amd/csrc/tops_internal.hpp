@@ -20,12 +20,14 @@ constexpr double kEllB = 6356752.3142451794975639665996337;  // cuConstants.cuh:
 constexpr int kLutRows = 2048;                    // Interval + 1, Constants.h:9
 constexpr int kAzShifts = 5;     // window offsets the shared azimuth pass takes
 constexpr int kAzShiftTaps = 16; // taps per shifted azimuth row (the window height)
-// range LUT row with its tap moments over u = tap - 5: 12 taps, m1 = sum k u
-// (a double over two floats), e0 = sum k - 1, m2 = sum k u^2 (64 bytes)
+// range LUT row with its tap moments over u = tap - 5: 12 taps, the mean mu =
+// sum k u / sum k (a double over two floats), e0 = sum k - 1, v = sum k (u -
+// mu)^2 (64 bytes)
 constexpr int kKrgxRow = 16;
-// e0 is held as a float: for |e0| up to this its rounding moves a phase of
-// 1e4 revolutions by 6e-10
-constexpr double kUnitSum = 1e-6;
+// rows of a table whose phase may be formed from its moments: sums within 1e-6 of
+// 1, which the float e0 holds to 2^-52 (the sums of 12 floats below 1 hardly
+// need more), second and third moments about the mean up to 1
+constexpr double kUnitSum = 1e-6, kUnitSumRounding = 0x1p-52;
 constexpr int kInterval = 2047;
 constexpr int kTaps = 12;                         // Main.cpp:75, 113
 constexpr int kHalf = kTaps / 2 - 1;              // c_Npoints2m1
@@ -91,7 +93,7 @@ struct tops_ctx {
     double* d_mom = nullptr;    // [2048 x 4] azimuth LUT moments M0 M1 M2 0
     float* d_kaz_sh = nullptr;  // [5 x 2048 x 16] azimuth rows shifted by 0..4 taps in 16
     float* d_krgx = nullptr;    // [2048 x kKrgxRow] range LUT rows with their moments
-    int krg_unit = 0;           // every range row sums to 1 within kUnitSum
+    int krg_unit = 0;           // every range row is as kUnitSum says
     int npoints = 12;
     tops::Scratch scratch;      // FP64 baseline intermediates
 };

@@ -110,3 +110,23 @@ def test_phase_arrays_that_are_not_finite(tops, orc, dev, d, rate, bad):
     assert 0 < lost.sum() <= 13 * 150
     assert np.array_equal(~np.isfinite(got), lost)
     assert rel_err(got[~lost], ref[~lost]) <= TOL
+
+
+def test_fitted_phase_rounds_like_the_sum(tops, orc, dev, d):
+    """The phase fitted over a strip's columns against the FP64 sum of its 12
+    columns, which one range row whose taps sum to 1 + 4e-6 makes the walker take:
+    the RMS error of the samples must be the same within 0.3 %.  The reference
+    time bends the phase by 2.1e-8 rad (1.4e-8 RMS) from a quadratic over 64
+    columns, which would be 0.7 % of the samples' 1.16e-7 if it were left out."""
+    kt, tref, fdc, krg = _arrays(d, "smooth")
+    bend = 2.4e-8 / (2 * np.pi * np.abs(kt * tref).mean() * 0.38 * 30.0 ** 3)
+    bend = bend * (np.arange(len(kt)) - 100.0) ** 3
+    tref, fdc = tref + bend, fdc + kt * bend   # kt tref - fdc stays
+    uneven = np.array(krg, np.float32).reshape(-1, 12)
+    uneven[1023] *= np.float32(1 + 4e-6)
+    rms = []
+    for k in (krg, uneven.reshape(np.shape(krg))):
+        got, ref = _both(tops, orc, dev, d, 400, 417, 68, 1.0, 2e-4, 31.3, (kt, tref, fdc, k))
+        rms.append(float(np.sqrt(np.mean(np.abs(got - ref) ** 2) / np.mean(np.abs(ref) ** 2))))
+    print(f"  RMS error: fitted {rms[0]:.5e}, summed {rms[1]:.5e}", flush=True)
+    assert rms[0] <= 1.003 * rms[1]
