@@ -162,11 +162,12 @@ __device__ __forceinline__ tops_cf32 interior_direct(const tops_ci16* slave, con
     return reramp(sr, si, phi);
 }
 
-// exp(j ph): the phase goes to half revolutions, where the reduction is exact
+// exp(j ph): reduced to [-pi, pi] with one rounding of 2 pi, then in half
+// revolutions, where the function's own reduction is exact
 __device__ __forceinline__ void phasor(double ph, double& re, double& im)
 {
-    const double t = ph * kInvTwoPi;
-    sincospi(2.0 * (t - rint(t)), &im, &re);
+    const double r = fma(-rint(ph * kInvTwoPi), kTwoPi, ph);
+    sincospi(r * (2.0 * kInvTwoPi), &im, &re);
 }
 
 // Column state of one lane: deramp recurrence along its slave column, with
