@@ -80,15 +80,6 @@ constexpr int WK_OUT = 52;
 constexpr int WK_WIN = 16;     // register window rows
 constexpr int kWalkWavesPerSimd = 3;   // occupancy the walker is compiled for
 
-__device__ inline void load_taps(const float* lut, int row, float k[kTaps])
-{
-    const float4* q = reinterpret_cast<const float4*>(lut + row * kTaps);
-    float4 a = q[0], b = q[1], c = q[2];
-    k[0] = a.x; k[1] = a.y; k[2] = a.z; k[3] = a.w;
-    k[4] = b.x; k[5] = b.y; k[6] = b.z; k[7] = b.w;
-    k[8] = c.x; k[9] = c.y; k[10] = c.z; k[11] = c.w;
-}
-
 // out = (sr + j si) * exp(-j phi).  The phase goes to revolutions and is
 // reduced to [-1/2, 1/2] in FP64; the hardware sine and cosine take
 // revolutions directly (absolute error about 1.3e-7 on that interval).
