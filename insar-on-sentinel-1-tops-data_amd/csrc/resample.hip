@@ -173,6 +173,7 @@ int launch_resample_fp64(tops_ctx* ctx, const ResampleParams& p, hipStream_t s)
 
 constexpr int WK_GROUP = 4;           // output rows per group (one matrix-instruction block)
 constexpr int WK_SLOTS = 2;           // azimuth keys per row and round
+constexpr int WK_LONG = 20;           // lines of the window where lines do not advance evenly
 // What the fitted phase may leave out: 2^-32 rad and 2^-47 of the size of the
 // phase's terms, a few roundings of the FP64 sum it takes the place of, and
 // never more than half an ulp of an FP32 sample of magnitude 1
@@ -278,22 +279,23 @@ typedef float MfmaAcc __attribute__((ext_vector_type(4)));
 // one column per lane, which is the walker's own layout.  Each step is an
 // FP32 fused multiply-add per element in line order, bit-equal to the
 // scalar-tap chain fmaf(tap, win, acc).
-template <int K, int S>
+// (lines 16 on of a longer window in a second register)
+template <int K, int S, int N, int T>
 struct AzStep {
-    __device__ __forceinline__ static void run(const WinRow (&win)[WK_WIN], const float (&wt)[WK_SLOTS],
+    __device__ __forceinline__ static void run(const WinRow (&win)[N], const float (&wt)[T][WK_SLOTS],
                                                MfmaAcc (&re)[S], MfmaAcc (&im)[S])
     {
-        AzStep<K - 1, S>::run(win, wt, re, im);
+        AzStep<K - 1, S, N, T>::run(win, wt, re, im);
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            re[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(wt[s], win_re(win[K]), re[s], 4, K, 0);
-            im[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(wt[s], win_im(win[K]), im[s], 4, K, 0);
+            re[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(wt[K / 16][s], win_re(win[K]), re[s], 4, K % 16, 0);
+            im[s] = __builtin_amdgcn_mfma_f32_4x4x1f32(wt[K / 16][s], win_im(win[K]), im[s], 4, K % 16, 0);
         }
     }
 };
-template <int S>
-struct AzStep<-1, S> {
-    __device__ __forceinline__ static void run(const WinRow (&)[WK_WIN], const float (&)[WK_SLOTS],
+template <int S, int N, int T>
+struct AzStep<-1, S, N, T> {
+    __device__ __forceinline__ static void run(const WinRow (&)[N], const float (&)[T][WK_SLOTS],
                                                MfmaAcc (&)[S], MfmaAcc (&)[S]) {}
 };
 
@@ -333,16 +335,18 @@ __device__ __forceinline__ int by_row(int k0, int k1, int k2, int k3, bool b0, b
 // FP64 phases per column.  kEven: the slave line advances by about one a row
 // and hardly along it, so that the window slides by 4 lines from group to group
 // and reaches all of a group's keys; the few outputs it does not reach are left
-// to the direct path.  Otherwise it slides by any number of lines, and to
-// further positions for keys it does not reach: that handling costs the even
-// rows 4 to 6 % (1500 x 21000: 232 us and 246).
+// to the direct path.  Otherwise the window is 4 lines longer, slides by any
+// number of lines, and to further positions for keys it does not reach: that
+// would cost even rows 10 % (1500 x 12000: 163 us and 179).
 template <bool kSmooth, bool kEven>
 __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r0, int r1,
                                           int ucol0, ColumnWalker& w, WalkLds& sm)
 {
     constexpr int G = WK_GROUP;
     constexpr int S = kSmooth ? WK_SLOTS : 1;   // azimuth keys per row and round
-    constexpr int kReach = kAzShifts - 1;       // lines past the window's first a key may start at
+    constexpr int N = kEven ? WK_WIN : WK_LONG;  // lines of the window
+    constexpr int kReach = N - kTaps;           // lines past the window's first a key may start at
+    static_assert(kAzShifts == WK_WIN - kTaps + 1, "the table's tap offsets");
     constexpr int kWaveShr1 = 0x138;            // DPP: the value of the lane to the left
     constexpr int kMaxSlide = 20;               // lines the window slides rather than start anew
     constexpr int kMaxMoves = 16;               // window positions after a group's first
@@ -361,7 +365,7 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
     const int xn = min(ucol0 + 64 - kTaps + kHalf, p.sb[1] - kHalf - 2) - xlo;
     const bool none = yn < 0 || xn < 0;
     const float2* u0 = &sm.u[0][none ? 0 : xlo - kHalf - ucol0];
-    WinRow win[WK_WIN];
+    WinRow win[N];
     int wbase = INT_MIN;           // absolute slave line held in win[0]
     bool late = false;             // outputs are marked for the direct path (uniform)
     // A group takes one round of up to S keys per row, or further rounds
@@ -471,7 +475,8 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             // row is served by its first slot.
             // (no head left reads lane 63, which owns no output)
             int kq[G][S];
-            const int lim = (wline + kReach) << 11 | (kLutRows - 1);
+            // (no line reaches kMaxSlaveLine)
+            const int lim = min(wline + kReach, kMaxSlaveLine - 1) << 11 | (kLutRows - 1);
 #pragma unroll
             for (int i = 0; i < G; i++) {
 #pragma unroll
@@ -490,13 +495,19 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             // window line k (the key's 12 taps pre-shifted by its line
             // offset, zeros elsewhere)
             int kr[S];
-            float wt[WK_SLOTS];
+            float wt[kEven ? 1 : 2][WK_SLOTS];
 #pragma unroll
             for (int s = 0; s < S; s++) {
                 kr[s] = by_row(kq[0][s], kq[1][s], kq[2][s], kq[3][s], b0, b1);
                 if (kr[s] < 0) kr[s] = wline << 11;
-                wt[s] = p.kaz_sh[((((kr[s] >> 11) - wline) * kLutRows + (kr[s] & (kLutRows - 1)))
-                                  * kAzShiftTaps) + (lane >> 2)];
+                const int o = (kr[s] >> 11) - wline, row = kr[s] & (kLutRows - 1);
+                if constexpr (kEven) {
+                    wt[0][s] = p.kaz_sh[(o * kLutRows + row) * kAzShiftTaps + (lane >> 2)];
+                } else {
+                    const int k0 = (lane >> 2) - o, k1 = k0 + 16;
+                    wt[0][s] = (unsigned)k0 < (unsigned)kTaps ? p.kaz[row * kTaps + k0] : 0.0f;
+                    wt[1][s] = (unsigned)k1 < (unsigned)kTaps ? p.kaz[row * kTaps + k1] : 0.0f;
+                }
             }
             float4 tap[2][4];
             auto load_range = [&](int i) {
@@ -510,11 +521,11 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             if constexpr (!kEven) {
                 if (__builtin_expect(slide < 0, 0)) {
                     w.anchor(p, wbase, sm.abc[0][lane], sm.abc[1][lane], sm.abc[2][lane]);
-                    int raw[WK_WIN];
+                    int raw[N];
 #pragma unroll
-                    for (int k = 0; k < WK_WIN; k++) raw[k] = w.fetch(p, wbase + k);
+                    for (int k = 0; k < N; k++) raw[k] = w.fetch(p, wbase + k);
 #pragma unroll
-                    for (int k = 0; k < WK_WIN; k++) win[k] = win_pack(w.deramp(raw[k]));
+                    for (int k = 0; k < N; k++) win[k] = win_pack(w.deramp(raw[k]));
                     w.prefetch(p);
                 } else {
                     for (; slide > 0; slide--) slide4(win, w, p);
@@ -543,7 +554,7 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
             if (kSmooth && second) {
                 // (four independent chains: no wait between dependent steps)
                 MfmaAcc re[2] = {}, im[2] = {};
-                AzStep<WK_WIN - 1, 2>::run(win, wt, re, im);
+                AzStep<N - 1, 2, N, kEven ? 1 : 2>::run(win, wt, re, im);
 #pragma unroll
                 for (int i = 0; i < G; i++) {
                     sm.u[i * S][lane] = make_float2(re[0][i], im[0][i]);
@@ -551,7 +562,7 @@ __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r
                 }
             } else {
                 MfmaAcc re[1] = {}, im[1] = {};
-                AzStep<WK_WIN - 1, 1>::run(win, wt, re, im);
+                AzStep<N - 1, 1, N, kEven ? 1 : 2>::run(win, wt, re, im);
 #pragma unroll
                 for (int i = 0; i < G; i++) sm.u[i * S][lane] = make_float2(re[0][i], im[0][i]);
             }
@@ -946,10 +957,11 @@ static StripHeights resample_heights(const int* lines, const int* pixels, int n)
 // anew at most every 8 groups, and 4 rows of a strip spread over at most 4
 // lines.  Both slopes are linear: their extremes are at the box's corners.  A
 // false comparison, as of NaN, takes the other form, which serves everything.
-// (1500 x 12000, this form against the other, us: 1 line a row 160 / 168, 0.98
-// 150 / 155, 1.02 148 / 149, 0.95 154 / 151, 0.9 159 / 151, 0.8 174 / 153, 0.5 191
-// / 148, 2 2560 / 222; lines a column 0.018 2260 / 2444, 0.025 3200 / 2520.  The
-// walker of one row at a time: 200 at 1, 177 at 0.5, 192 at 2 lines a row.)
+// (1500 x 12000, this form against the other, us: 1 line a row 163 / 179, 0.98 161
+// / 167, 0.95 156 / 158, 0.9 160 / 155, 0.8 174 / 151, 0.5 191 / 148, 2 2560 / 167;
+// lines a column 0.018 2263 / 2530, 0.025 3200 / 2525.  The walker of one row at a
+// time: 200 at 1, 170 at 0.5, 192 at 2, 206 at 3 lines a row, where the other form
+// takes two window positions a group, 246.)
 bool resample_even(const ResampleParams& p)
 {
     const double per_row = 4.0 / (p.mb[3] - p.mb[2]), per_col = 4.0 / (p.mb[1] - p.mb[0]);

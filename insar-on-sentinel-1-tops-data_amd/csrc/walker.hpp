@@ -269,9 +269,8 @@ __device__ __forceinline__ float win_im(WinRow w) { return __uint_as_float((unsi
 // in the registers the raw values held, and stay in flight until the next
 // slide.  (Requested earlier, the compiler copies the landing registers at
 // once, which waits for the loads.)
-template <typename Win>
-__device__ __forceinline__ void slide4(Win (&win)[WK_WIN], ColumnWalker& w,
-                                       const ResampleParams& p)
+template <int N>
+__device__ __forceinline__ void slide4(WinRow (&win)[N], ColumnWalker& w, const ResampleParams& p)
 {
     float2 v[4];
 #pragma unroll
@@ -280,24 +279,23 @@ __device__ __forceinline__ void slide4(Win (&win)[WK_WIN], ColumnWalker& w,
                  "+v"(v[2].y), "+v"(v[3].x), "+v"(v[3].y)::"memory");
     w.prefetch(p, 4);   // the 4 lines after the ones unpacked
 #pragma unroll
-    for (int k = 0; k < WK_WIN - 4; k++) win[k] = win[k + 4];
+    for (int k = 0; k < N - 4; k++) win[k] = win[k + 4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) win[WK_WIN - 4 + k] = win_pack(w.deramp(v[k]));
+    for (int k = 0; k < 4; k++) win[N - 4 + k] = win_pack(w.deramp(v[k]));
 }
 
 // Slide a window by one row (rare: the pending lines move up, which waits for
 // them)
-template <typename Win>
-__device__ __forceinline__ void slide1(Win (&win)[WK_WIN], ColumnWalker& w,
-                                       const ResampleParams& p)
+template <int N>
+__device__ __forceinline__ void slide1(WinRow (&win)[N], ColumnWalker& w, const ResampleParams& p)
 {
     const int raw = w.pend[0];
 #pragma unroll
     for (int k = 0; k < 3; k++) w.pend[k] = w.pend[k + 1];
     w.pend[3] = w.fetch(p, w.ynext + 4);
 #pragma unroll
-    for (int k = 0; k < WK_WIN - 1; k++) win[k] = win[k + 1];
-    win[WK_WIN - 1] = win_pack(w.deramp(raw));
+    for (int k = 0; k < N - 1; k++) win[k] = win[k + 1];
+    win[N - 1] = win_pack(w.deramp(raw));
 }
 
 // read-only tables addressed with wave-uniform indices
