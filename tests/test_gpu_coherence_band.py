@@ -28,6 +28,7 @@ def _inputs(h, w, seed):
 
 # (window lines, samples), (lines before, samples before), (lines, samples); the
 # rasters have more tiles of 16 x 64 than run at once, so they take the bands
+# (3 x 10 on 700 x 1019 has 704, which still run at once: the tiles)
 @pytest.mark.parametrize("win,off,shape", [
     ((2, 4), (0, 1), (1301, 1000)),
     ((2, 8), (1, 7), (33, 25001)),
@@ -80,3 +81,22 @@ def test_band_split_independent(tops, dev, wa, wr):
 
     whole, part = run(M, S, h), run(M[cut:], S[cut:], h - cut)
     assert np.array_equal(whole[cut + wa:], part[wa:])
+
+
+@pytest.mark.parametrize("shape", [(1100, 1019), (33, 25001), (1487, 769)])
+def test_default_window_in_bands(tops, orc, dev, shape):
+    """The 3 x 10 window at its default centre on rasters of more than 4 tiles of
+    16 x 64 per CU."""
+    N = tops.native
+    L = N.load()
+    h, w = shape
+    assert -(-h // 16) * -(-w // 64) > 4 * dev.torch.cuda.get_device_properties(
+        0).multi_processor_count
+    M, S = _inputs(h, w, h)
+    ref = orc.coherence(M, S.astype(np.complex128), 4, 1, 10, 3)
+    dm, ds, dc = dev.put(M), dev.put(S), dev.empty(h * w * 4)
+    N.check(L.tops_coherence(dm.data_ptr(), ds.data_ptr(), w, h, 4, 1, 10, 3, dc.data_ptr(), 0,
+                             None))
+    got = dev.get(dc, np.float32, (h, w))
+    assert not got[np.abs(S) < 0.0009].any()
+    assert float(np.max(np.abs(got - ref))) <= TOL

@@ -12,8 +12,9 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# fifth: metres per (10 s)^5; its polynomial range is (1e-11 / fifth)^0.2 x 10 s:
-# 6e-3 s at 1e4, 1.6e-3 s at 1e7, where a tile of 1 arcsec reaches 1e-2 s
+# fifth: metres per (10 s)^5; the polynomial's range is (2e-12 / fifth)^0.25 x 10 s,
+# where its velocity is within 1e-12 m/s: 1.2e-3 s at 1e4, 2.1e-4 s at 1e7, where a
+# tile of 1 arcsec reaches 1e-2 s (test_tiles_in_part: 1.2e-2 s at 1, 6.7e-3 at 10)
 @pytest.mark.parametrize("fifth", [0.0, 1e4, 1e7])
 @pytest.mark.parametrize("rows,cols", [(1, 1), (4, 64), (5, 65), (61, 333)])
 def test_orbit_polynomials(tops, orc, dev, fifth, rows, cols):
@@ -56,3 +57,10 @@ def test_orbit_polynomials(tops, orc, dev, fifth, rows, cols):
         ep = float(np.max(np.abs(got[2 * k + 1] - pix)))
         print(f"  {rows} x {cols}, fifth {fifth:g}: line {el:.2e}, pixel {ep:.2e}", flush=True)
         assert el <= 1e-4 and ep <= 1e-3
+
+
+@pytest.mark.parametrize("fifth", [1.0, 3.0, 10.0])
+def test_tiles_in_part(tops, orc, dev, fifth):
+    """Fifth-order terms whose range ends inside a tile: some of its posts take
+    the polynomial, some the full iteration."""
+    test_orbit_polynomials(tops, orc, dev, fifth, 61, 333)

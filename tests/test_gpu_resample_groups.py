@@ -1,7 +1,7 @@
 """The resample walker's row groups against the FP64 oracle
-(DerampAndResample.cu:348-520 semantics): strips that end inside a group, at a
-row table's edge or one row past it, several azimuth keys a row, and the two
-forms of the phase.  Samples agree to max|dz|/RMS|z| <= 1e-5, the tolerance of
+(DerampAndResample.cu:348-520 semantics) in launches so small that every strip is
+one group: groups of fewer rows, several azimuth keys a row, and the two forms of
+the phase.  (Strips of many groups: test_gpu_resample_walk.py.)  Samples agree to max|dz|/RMS|z| <= 1e-5, the tolerance of
 the resampled samples everywhere: FP32 sums of 24 terms of magnitude up to
 the largest sample reach 24 * 2^-24 * max/RMS, about 6e-6."""
 import ctypes as C
@@ -47,7 +47,7 @@ def d(tops, orc):
 
 
 # (rows, columns) of the top-left of the burst that are resampled at about one
-# slave line a row: one group less a row .. past a 32-row position table
+# slave line a row: part of a group .. 17 of them one below the other
 @pytest.mark.parametrize("rows,cols", [(1, 52), (3, 53), (5, 64), (31, 105), (33, 157), (67, 300)])
 @pytest.mark.parametrize("form", ["smooth", "rough", "taps"])
 def test_groups(tops, orc, dev, d, rows, cols, form):

@@ -1,6 +1,7 @@
-"""Host buffers of the reference-style calls: sizes about the staging chunks
-(4 MiB, four in flight), unaligned, pinned and pageable, from several threads
-at once, give the bytes that the device entry points give."""
+"""Host buffers of the reference-style calls: sizes about the smallest staging
+chunk (4 MiB; an eighth of larger uploads, 32 MiB for downloads, two chunks in
+flight), unaligned, pinned and pageable, from several threads at once, give the
+bytes that the device entry points give."""
 import ctypes as C
 import threading
 
@@ -18,8 +19,9 @@ def _case(tops, orc):
     return m, kt[0], tref[0], fdc[0], kaz, krg
 
 
-# lines x 1024 samples: the slave (4 bytes a sample) just under, at and over one
-# chunk, and over the four workers' first chunks; the output has twice the bytes
+# lines x 1024 samples: the slave (4 bytes a sample) just under, at and over 4
+# MiB, the smallest copy that is staged, and of five chunks; the output has twice
+# the bytes, up to a chunk and a part of the next
 @pytest.mark.parametrize("lines", [1023, 1024, 1025, 5121])
 @pytest.mark.parametrize("kind", ["pageable", "unaligned", "pinned"])
 def test_sizes_and_kinds(tops, orc, dev, lines, kind):
@@ -109,3 +111,28 @@ def test_sums_from_several_threads(tops, dev):
     for t in th:
         t.join()
     assert not bad
+
+
+# bytes: chunks of an eighth up to 256 MiB, then of 32 MiB; downloads in 32 MiB
+# chunks, whose two buffers are taken in turn
+@pytest.mark.parametrize("nbytes", [(4 << 20) + 4, (70 << 20) + 12, (256 << 20) - 8,
+                                    (256 << 20) + 8, (300 << 20) + 20])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_staged_copies(tops, dev, nbytes, offset):
+    """The staging layer's own copies, up and down, of sizes past every change of
+    its chunks and with a part of a chunk left."""
+    L = tops.native.load()
+    up, down = (getattr(L, f"_ZN4tops{len(n)}{n}{a}") for n, a in
+                (("staged_upload", "EPvPKvm"), ("staged_download", "EPvPKvm")))
+    for f in (up, down):
+        f.argtypes, f.restype = [C.c_void_p, C.c_void_p, C.c_size_t], C.c_int
+    raw = np.empty(nbytes + 64, np.uint8)
+    src = raw[offset:offset + nbytes]
+    src[:] = np.arange(nbytes // 4, dtype=np.uint32).view(np.uint8)
+    d = dev.empty(nbytes)
+    assert up(d.data_ptr(), src.ctypes.data, nbytes) == 0
+    got = np.zeros(nbytes + 64, np.uint8)
+    assert down(got[offset:].ctypes.data, d.data_ptr(), nbytes) == 0
+    assert np.array_equal(got[offset:offset + nbytes], src)
+    assert not got[:offset].any() and not got[offset + nbytes:].any()
+    assert np.array_equal(d.cpu().numpy(), src)
