@@ -198,6 +198,15 @@ __device__ __forceinline__ double lane_value(double v, int lane)
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                             __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
+// 1 / n from the hardware's estimate (23 bits) in two Newton steps
+__device__ __forceinline__ double recip(int n)
+{
+    const double x = (double)n;
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
 // Fits the strip's phase coefficients into sm.fit, each the cubic through its
 // values at four columns near the Chebyshev places (false: not smooth enough on
 // the slave box's lines, which hold every interior output's).
@@ -213,16 +222,17 @@ __device__ __forceinline__ bool fit_phase(const ResampleParams& p, WalkLds& sm, 
     // the column of t = 0, from the places
     const double a0 = (double)(l0 + kHalf - t0), a1 = (double)(l0 + kHalf - t1);
     const double a2 = (double)(l0 + kHalf - t2);
-    const double ro = 1.0 / (double)(t1 - t0), ri = 1.0 / (double)(t2 - t1);
-    const double r2 = 1.0 / (double)(t2 - t0), r3 = 1.0 / (double)(t3 - t0);
+    const double ro = recip(t1 - t0), ri = recip(t2 - t1), r2 = recip(t2 - t0), r3 = recip(t3 - t0);
     // What the fit leaves out of the phase is a quadratic of the line: its values
     // at the ends and the middle of the box bound it within a factor 1.25 in
-    // between.  It is this lane's residual, the third moment of the taps (below
-    // 1) times the cubic's leading coefficient, and the rounding of their second.
+    // between.  It is each lane's residual, and the third moment of the taps
+    // (below 1) times the cubic's leading coefficient and the rounding of their
+    // second, which are the strip's: a lane takes them at one of the three lines.
     const double y0 = (double)p.sb[2] - (double)p.first_line;
-    const double y2 = (double)p.sb[3] - (double)p.first_line;
-    const double y[3] = {y0, 0.5 * (y0 + y2), y2}, ym = fmax(fabs(y0), fabs(y2));
-    double e[3] = {}, third[3] = {}, second[3] = {}, size = 0.0, yk[3] = {1.0, 1.0, 1.0}, ymk = 1.0;
+    const double y2 = (double)p.sb[3] - (double)p.first_line, y1 = 0.5 * (y0 + y2);
+    const double ym = fmax(fabs(y0), fabs(y2)), yl = lane & 2 ? y2 : lane & 1 ? y1 : y0;
+    double e0 = 0.0, e1 = 0.0, e2 = 0.0, third = 0.0, second = 0.0, size = 0.0;
+    double s0 = 1.0, s1 = 1.0, s2 = 1.0, sl = 1.0, sz = 1.0;
 #pragma unroll 1
     for (int k = 0; k < 3; k++) {
         const double v = sm.abc[k][lane];
@@ -237,25 +247,24 @@ __device__ __forceinline__ bool fit_phase(const ResampleParams& p, WalkLds& sm, 
         sm.fit[k][2] = c2 * kInvTwoPi;
         sm.fit[k][3] = d3 * kInvTwoPi;
         const double res = v - fma(x0, fma(x1, fma(x2, d3, d02), d01), f0);
-        size = fma(ymk, fabs(v), size);
-        ymk *= ym;
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            e[j] = fma(yk[j], res, e[j]);
-            third[j] = fma(yk[j], d3, third[j]);
-            second[j] = fma(yk[j], c2, second[j]);
-            yk[j] *= y[j];
-        }
+        e0 = fma(s0, res, e0);
+        e1 = fma(s1, res, e1);
+        e2 = fma(s2, res, e2);
+        third = fma(sl, d3, third);
+        second = fma(sl, c2, second);
+        size = fma(sz, fabs(v), size);
+        s0 *= y0;
+        s1 *= y1;
+        s2 *= y2;
+        sl *= yl;
+        sz *= ym;
     }
-    double r = 0.0, nan = 0.0;
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        r = fmax(r, fabs(e[j]) + fabs(third[j]) + 0x1p-24 * fabs(second[j]));
-        nan += 0.0 * (e[j] + third[j] + second[j]);
-    }
-    // (fmax drops a NaN: the sum keeps it, and a NaN fails the comparison)
     const double tol = fmin(kSmoothTol + kSmoothRel * size, kSmoothMax);
-    return __ballot(lane >= l0 && lane <= l1 && !(1.25 * r + nan <= tol)) == 0ull;
+    const double r = 2.5 * fmax(fmax(fabs(e0), fmax(fabs(e1), fabs(e2))),
+                                fma(0x1p-24, fabs(second), fabs(third)));
+    // (fmax drops a NaN: the sum keeps it, and a NaN fails the comparison)
+    const double nan = 0.0 * (e0 + e1 + e2 + third + second);
+    return __ballot(lane >= l0 && lane <= l1 && !(r + nan <= tol)) == 0ull;
 }
 
 // The mark of an interior output left to the direct path, in its place in the
