@@ -346,7 +346,7 @@ __device__ __forceinline__ int by_row(int k0, int k1, int k2, int k3, bool b0, b
 // and reaches all of a group's keys; the few outputs it does not reach are left
 // to the direct path.  Otherwise the window is 4 lines longer, slides by any
 // number of lines, and to further positions for keys it does not reach: that
-// would cost even rows 10 % (1500 x 12000: 163 us and 179).
+// would cost even rows 8 % (1500 x 12000: 164 us and 177).
 template <bool kSmooth, bool kEven>
 __device__ __forceinline__ void walk_rows(const ResampleParams& p, int c0, int r0, int r1,
                                           int ucol0, ColumnWalker& w, WalkLds& sm)
@@ -962,15 +962,15 @@ static StripHeights resample_heights(const int* lines, const int* pixels, int n)
 }
 
 // Whether the walker's form for even positions serves an item: over the whole
-// box the slave line advances by 1 within 1/32 a row, so that the window starts
-// anew at most every 8 groups, and 4 rows of a strip spread over at most 4
+// box the slave line advances by 1 within 1/16 a row, so that the window starts
+// anew at most every fourth group, and 4 rows of a strip spread over at most 4
 // lines.  Both slopes are linear: their extremes are at the box's corners.  A
 // false comparison, as of NaN, takes the other form, which serves everything.
-// (1500 x 12000, this form against the other, us: 1 line a row 163 / 179, 0.98 161
-// / 167, 0.95 156 / 158, 0.9 160 / 155, 0.8 174 / 151, 0.5 191 / 148, 2 2560 / 167;
-// lines a column 0.018 2263 / 2530, 0.025 3200 / 2525.  The walker of one row at a
-// time: 200 at 1, 170 at 0.5, 192 at 2, 206 at 3 lines a row, where the other form
-// takes two window positions a group, 246.)
+// (1500 x 12000, this form against the other, us: 1 line a row 164 / 177, 0.95 164
+// / 167, 1.05 150 / 155, 0.9 169 / 162, 0.8 183 / 157, 0.5 188 / 150, 2 2570 / 166;
+// lines a column 0.018 2263 / 2526, 0.025 3211 / 2523.  The walker of one row at a
+// time: 202 at 1, 168 at 0.5, 192 at 2, and 206 at 3 lines a row, where the other
+// form takes two window positions a group, 245.)
 bool resample_even(const ResampleParams& p)
 {
     const double per_row = 4.0 / (p.mb[3] - p.mb[2]), per_col = 4.0 / (p.mb[1] - p.mb[0]);
@@ -979,7 +979,7 @@ bool resample_even(const ResampleParams& p)
         const double* c = p.cpm_az;
         const double rate = (c[1] + 2.0 * c[3] * ln + c[4] * pn) * per_row;
         const double shear = (c[2] + c[4] * ln + 2.0 * c[5] * pn) * per_col;
-        if (!(std::fabs(rate - 1.0) <= 1.0 / 32 &&
+        if (!(std::fabs(rate - 1.0) <= 1.0 / 16 &&
               (WK_GROUP - 1) * rate + WK_OUT * std::fabs(shear) <= kAzShifts - 1))
             return false;
     }
