@@ -48,3 +48,38 @@ def test_bands(tops, orc, dev, win, sizes, pixels):
     for i, k in enumerate(sizes):
         assert e[i] <= 0.25 + 1e-6 * k * pixels
         assert k > 0 or not got[i].any()
+
+
+@pytest.mark.parametrize("win", [(2, 8), (3, 10), (5, 20), (8, 32)])
+def test_bands_sum_to_rounding(tops, orc, dev, win):
+    """Coherent samples throughout (0.95, none near a threshold, none zero): the
+    sums differ from the oracle's by the rounding of the unit phasors alone, at
+    most 2^-22 each (a reciprocal square root good to an ulp and a product), and
+    as roundings of either sign by about the square root of their number: 32 times
+    that is allowed."""
+    N = tops.native
+    L = N.load()
+    wa, wr = win
+    sizes, pixels = [97, 60, 33], 15002
+    rng = np.random.default_rng(wa)
+    n = sum(sizes)
+    M, S = [], []
+    for k in range(2):
+        m = np.round(rng.normal(0, 300, (n, pixels, 2))).astype(np.int16)
+        m[(m == 0).all(-1)] = 1
+        mc = m[..., 0] + 1j * m[..., 1]
+        th = 0.3 + 0.2 * k + 1e-3 * np.arange(pixels) * (1 - 2 * k)
+        S.append((mc * np.exp(1j * th) + rng.normal(0, 60, (n, pixels))
+                  + 1j * rng.normal(0, 60, (n, pixels))).astype(np.complex64))
+        M.append(m)
+    args = (M[0], M[1], S[0], S[1])
+    sz = np.array(sizes, np.int32)
+    d = [dev.put(np.ascontiguousarray(a)) for a in args]
+    shifts, sums = np.zeros(len(sz)), np.zeros(2 * len(sz))
+    N.check(L.tops_esd_shifts(*[x.data_ptr() for x in d], N.ptr(sz, C.c_int), len(sz), pixels, wa,
+                              wr, 0.3, 4500.0, 2e-3, N.ptr(shifts), N.ptr(sums), None))
+    _, rsums = orc.esd(*args, sz, pixels, wa, wr, 0.3, 4500.0, 2e-3)
+    e = np.abs(sums.reshape(-1, 2) - np.asarray(rsums).reshape(-1, 2)).max(axis=1)
+    bound = 32 * 2.0 ** -22 * np.sqrt(sz.astype(float) * pixels)
+    print(f"  {wa} x {wr}: sums |d| {e}, allowed {bound}", flush=True)
+    assert np.all(e <= bound)
