@@ -15,6 +15,10 @@
  *     once, each thread with its own status; a context (tops_ctx) may be
  *     shared, while a plan (tops_plan) and the fixed scratch of
  *     tops_esd_shifts_noalloc serve one call at a time;
+ *   - kept per device between calls: 64 MiB of pinned memory from the first
+ *     copy of over 4 MiB of pageable memory on, whose copies take turns, and
+ *     up to 4 idle scratch blocks of at most 8 MiB of tops_esd_shifts and
+ *     tops_geocoreg, which tops_ctx_destroy gives back;
  *   - device buffers returned by DerampDemodResample_ESD/ResampleFirstBurst
  *     are dense [rows x cols] (pitch = cols) and are released by the
  *     CoherenceEst* call that consumes them, as in the reference.

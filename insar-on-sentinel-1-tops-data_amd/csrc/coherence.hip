@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(256) coherence_batch_kernel(const CohItem* ite
 
 // ---- band form (coherence_band.hpp) --------------------------------------
 // Workgroups of 256 threads, as many per CU as the registers allow (waves per
-// SIMD): 4 for 2 and 3 lines (82 and 96 VGPRs), 3 for 4 to 7 (113 to 160; 4
+// SIMD): 4 for 2 and 3 lines (82 and 97 VGPRs), 3 for 4 to 7 (113 to 161; 4
 // lines at 4 waves 123 us against 114 on 1487 x 24491, 7 x 20 at 2 waves 125 us
 // against 110 on 1500 x 21000), 2 above (205).
 __host__ __device__ constexpr int band_waves(int win_az)

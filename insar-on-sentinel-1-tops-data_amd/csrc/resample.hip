@@ -130,8 +130,8 @@ int launch_resample_fp64(tops_ctx* ctx, const ResampleParams& p, hipStream_t s)
 // One 64-lane workgroup owns a strip of output rows x WK_OUT output columns.
 // Lane l is bound to slave column ucol0 + l for the whole strip and walks it
 // in groups of output rows:
-//   * it keeps the deramped slave samples of rows wbase..wbase+15 of its
-//     column in registers; new rows are deramped on arrival with an FP64
+//   * it keeps the deramped slave samples of rows wbase..wbase+15 (+19 where
+//     lines advance unevenly) of its column in registers; new rows are deramped on arrival with an FP64
 //     phasor recurrence along the column (exp(j phi) is advanced by
 //     exp(j (b + c (2y+1))), which is advanced by exp(j 2c)), anchored with
 //     an FP64 sincos at the strip start and after a resync;
@@ -930,9 +930,7 @@ StripHeights resample_heights_of(int tall, const int* lines, const int* pixels, 
 // height that does not (700 x 9000: 69 us at 28, 60 at 32).  Few rows fill the
 // slots once, in strips of 8 rows (512 x 2048: 24 us at 8, 26 at 12), or of 4,
 // one group, where those all run at once: a wave is a chain of its groups (130 x
-// 1000: 13.9 us, 21.0 at 8; 300 x 2000 17.8, 20.4; 130 x 360, whose phase arrays
-// bend too much over 64 columns for the fit and whose rows hold many keys, 35 us,
-// 59 at 8, 40 with the row-at-a-time walker).
+// 1000: 13.9 us, 21.0 at 8; 300 x 2000 17.8, 20.4).
 // One height for 6 rounds against this: 1500 x 21000 250 us -> 234, 1487 x
 // 24491 289 -> 267, 1200 x 15000 152 -> 145, 700 x 9000 75 -> 60, 300 x 20000
 // 73 -> 62, 100 x 21000 32 -> 29.
